@@ -37,149 +37,22 @@
 // the sign rotated to the lowest bit so that both signs form one contiguous range); a pass of 32 tokens with any gate
 // outside that range (zeros, tinier, larger, inf, NaN -- the wave votes) reads the full table in global memory
 // instead.  Both give the same table entry, so the output does not depend on the path taken.
-// Other forms below, each with the same MFMA sequence per output element (so the same bits): the half-tile kernel
-// (256 tokens x 128 channels, three stages) for a problem's last partial round and for problems of fewer tiles than
-// CUs, the 128 x 192 tiles (one per CU) for such problems when they occupy more CUs than the half tiles would, and
-// the small-M form (M <= 32: one wave per 16 weight rows, the weight streamed once).
+// Other forms, each with the same MFMA sequence per output element (so the same bits): the small-M form below (M <= 32:
+// one wave per 16 weight rows, the weight streamed once) and the smaller tiles of gemm_tile.hip (a problem's last partial
+// round, and problems of too few 256 x 256 tiles for the CUs).
 #include <algorithm>
 
-#include "h3fp8_common.h"
+#include "gemm_core.h"
 
 namespace {
 
-using namespace h3;
-
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef unsigned int v2u32 __attribute__((ext_vector_type(2)));
+using namespace h3g;
 
 constexpr int BM = 256;          // tokens per block tile
 constexpr int BN = 256;          // weight rows per block tile
-constexpr int BK = 128;          // k per stage: 128-byte row pieces
-constexpr int ROWB = BK;         // bytes per LDS row
 constexpr int STAGE_BYTES = (BM + BN) * ROWB;   // 64 KiB
 constexpr int NSTAGE = 2;
 constexpr int A_REGION = BN * ROWB;             // activation rows start after the weight rows
-constexpr uint32_t OOB = 0x80000000u;         // an offset past every buffer's range: the load returns zeros
-
-enum Epi { EPI_PLAIN = 0, EPI_AMAX = 1, EPI_SWIGLU = 2 };
-
-struct GemmParams {
-    const uint8_t* a;          // [M, K] e4m3, row stride lda
-    const uint8_t* w;          // [Nw, K] e4m3, row stride ldw (Nw = N, or 2F for SwiGLU)
-    const float* sa;
-    const float* sb;
-    const void* bias;
-    void* y;                   // [M, N] (SwiGLU: [M, F])
-    float* row_amax;           // EPI_AMAX / EPI_SWIGLU (may be null for SwiGLU)
-    const uint16_t* silu;      // SwiGLU table
-    const uint16_t* silu_rot;  // its compact rotated-key copy (loaded into LDS)
-    int64_t lda, ldw, ldy;
-    int64_t sa_stride, sb_stride;
-    int M, N, K;               // SwiGLU: N = F (output width)
-    int w_rows;                // rows of w and entries of sb (N, or 2F for SwiGLU)
-    uint32_t a_bytes, w_bytes; // buffer ranges
-    uint32_t y_bytes;          // output range: ((M - 1) * ldy + N) * element size; stores past it are dropped
-    int tiles_m, tiles_n;
-    int group_m;
-    int tile_offset;           // grouped launches: first block of this problem
-    int half_first;            // half-tile launches: the first tile (in the full-tile order) they cover
-    int y_nt;                  // fp32 outputs: store non-temporally (the whole product is larger than the MALL)
-};
-
-// block index -> (tile_m, tile_n): XCD-contiguous ranges, then GROUP_M-row groups (column-major inside a group).
-__device__ __forceinline__ void tile_of(int b, int T, int tiles_m, int tiles_n, int group_m, int& tm, int& tn) {
-    const int xcd = b & 7, local = b >> 3;
-    const int per = T >> 3, rem = T & 7;
-    int lid = (xcd < rem) ? xcd * (per + 1) + local : rem * (per + 1) + (xcd - rem) * per + local;
-    const int in_group = group_m * tiles_n;
-    const int g = lid / in_group;
-    const int first = g * group_m;
-    const int gsz = min(tiles_m - first, group_m);
-    const int r = lid - g * in_group;
-    tm = first + r % gsz;
-    tn = r / gsz;
-}
-
-// LDS chunk swizzle (see the header): logical 16-byte chunk c of row r is stored at chunk c ^ swz(r).
-__device__ __forceinline__ int swz(int r) { return ((r >> 1) & 7) ^ ((r & 1) << 2); }
-
-// One 32 x 64 MFMA operand of k sub-step `sub`: lane l reads row (l & 31) of the tile, logical chunks 4 sub + 2h and
-// 4 sub + 2h + 1 (h = l >> 5).  Tile bases are multiples of 32 rows, so swz of the tile row equals swz of the LDS row.
-__device__ __forceinline__ v8i read_frag(const uint8_t* tile, int lane, int sub) {
-    const int row = lane & 31, h = lane >> 5;
-    const uint8_t* p = tile + row * ROWB;
-    const int s = swz(row);
-    const int c0 = 4 * sub + 2 * h;
-    const uint4 lo = *reinterpret_cast<const uint4*>(p + ((c0 ^ s) << 4));
-    const uint4 hi = *reinterpret_cast<const uint4*>(p + (((c0 + 1) ^ s) << 4));
-    v8i f;
-    f[0] = (int)lo.x; f[1] = (int)lo.y; f[2] = (int)lo.z; f[3] = (int)lo.w;
-    f[4] = (int)hi.x; f[5] = (int)hi.y; f[6] = (int)hi.z; f[7] = (int)hi.w;
-    return f;
-}
-
-__device__ __forceinline__ float load_bias(const void* bias, int n, int out_dt) {
-    uint16_t b = reinterpret_cast<const uint16_t*>(bias)[n];
-    return out_dt ? fp16_to_f32(b) : bf16_to_f32(b);
-}
-
-// s_waitcnt immediate for vmcnt(n) alone (gfx9 encoding: vmcnt[3:0] in bits 3:0, vmcnt[5:4] in bits 15:14, expcnt
-// and lgkmcnt left at their maxima).
-constexpr int vmcnt_imm(int n) { return (n & 0xf) | ((n >> 4) << 14) | (0x7 << 4) | (0xf << 8); }
-
-__device__ __forceinline__ void wait_vm0() { __builtin_amdgcn_s_waitcnt(vmcnt_imm(0)); }
-
-__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xc07f); }
-
-// Workgroup barrier without a memory-model fence: __syncthreads() would add a release fence that waits for every
-// in-flight LDS-DMA load (vmcnt(0)), including the k-steps still being prefetched.  The explicit vmcnt/lgkmcnt waits
-// before it carry the ordering; the "memory" clobber keeps the compiler from moving LDS accesses across it.
-__device__ __forceinline__ void barrier_nofence() { asm volatile("s_barrier" ::: "memory"); }
-
-// A buffer descriptor as four dwords (base, stride 0, num_records = byte range, gfx9 raw-buffer flags); loads at
-// offsets >= num_records return zeros.
-__device__ __forceinline__ v4u buffer_desc(const void* base, uint32_t bytes) {
-    const uint64_t b = reinterpret_cast<uint64_t>(base);
-    v4u d;
-    d[0] = __builtin_amdgcn_readfirstlane((uint32_t)b);
-    d[1] = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32) & 0xffffu);
-    d[2] = __builtin_amdgcn_readfirstlane(bytes);
-    d[3] = 0x00020000u;
-    return d;
-}
-
-// 16 bytes per lane from a buffer straight into LDS at lds_base + 16 * lane (buffer_load_dwordx4 ... lds).
-// Written as inline asm so that the compiler's wait-count pass does not track these loads: it cannot tell one LDS
-// stage from another and would wait for every in-flight load before each LDS read.  The kernel therefore places
-// every wait on these loads itself (wait_vm before the barrier that publishes a stage).
-__device__ __forceinline__ void dma16(v4u desc, uint32_t lds_base, uint32_t voff) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                 :
-                 : "s"(lds_base), "v"(voff), "s"(desc)
-                 : "memory", "m0");
-}
-
-// The same load with the non-temporal hint, for operands that stream through once.
-__device__ __forceinline__ void dma16_nt(v4u desc, uint32_t lds_base, uint32_t voff) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
-                 :
-                 : "s"(lds_base), "v"(voff), "s"(desc)
-                 : "memory", "m0");
-}
-
-__device__ __forceinline__ uint32_t lds_addr(const uint8_t* p) {
-    typedef const __attribute__((address_space(3))) uint8_t* lds_u8;
-    return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_u8)(p));
-}
-
-// 4 bytes per lane straight into LDS at lds_base + 4 * lane (buffer_load_dword ... lds); untracked like dma16.
-__device__ __forceinline__ void dma4(v4u desc, uint32_t lds_base, uint32_t voff) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds"
-                 :
-                 : "s"(lds_base), "v"(voff), "s"(desc)
-                 : "memory", "m0");
-}
-
 // ---- LDS layout of a workgroup ----
 //   kernel 2 (150.5 KiB of the 160 KiB):
 //   [0, 128 KiB)          two operand stages of 64 KiB (weight rows, then token rows, 128 bytes each)
@@ -487,43 +360,6 @@ __device__ __forceinline__ void kstep(uint8_t* lds, uint32_t lds0, int g, const 
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-}
-
-// Orders one wave's LDS accesses across its lanes: a lane's staging writes become visible to the other lanes' reads
-// that follow.  The wave's LDS accesses already complete in order, so this emits no wait; it is there for the compiler,
-// which under per-lane semantics may otherwise reorder or tail-duplicate lane-divergent writes past other lanes' reads
-// (the barrier is convergent: it cannot be moved into a divergent branch).
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// max(m, |lo half|, |hi half|) of a packed bf16 pair, as fp32 bit patterns (the row maximum of the fused quant).
-__device__ __forceinline__ uint32_t max_abs_bf16x2(uint32_t m, uint32_t p) {
-    const uint32_t lo = (p << 16) & 0x7fff0000u, hi = p & 0x7fff0000u;
-    m = m > lo ? m : lo;
-    return m > hi ? m : hi;
-}
-
-// The same for a packed fp16 pair: each half is widened to fp32 (exact) before its |.| bits are compared, so the row
-// maximum is the fp32 value of the largest rounded fp16 output (NaN patterns exceed every finite one, as above).
-__device__ __forceinline__ uint32_t max_abs_f16x2(uint32_t m, uint32_t p) {
-    const uint32_t lo = f2u(fp16_to_f32(p & 0xffffu)) & 0x7fffffffu, hi = f2u(fp16_to_f32(p >> 16)) & 0x7fffffffu;
-    m = m > lo ? m : lo;
-    return m > hi ? m : hi;
-}
-
-// Running maxima of |x| over packed bf16 pairs, one per 16-bit half: with the sign bit cleared, bf16 magnitudes order
-// as their bit patterns (NaN patterns above inf), so a pair costs one mask and one packed u16 max.  pk_max_f32 folds
-// the two halves into the fp32 bit pattern of the larger, the value max_abs_bf16x2 accumulates over the same pairs.
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ u16x2 max_abs_pk(u16x2 m, uint32_t p) {
-    return __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, p & 0x7fff7fffu));
-}
-__device__ __forceinline__ uint32_t pk_max_f32(u16x2 m) {
-    const uint32_t a = m[0], b = m[1];
-    return (a > b ? a : b) << 16;
 }
 
 // A +0 the compiler cannot see through, made once per epilogue: x + z turns -0 into +0 (round to nearest) and leaves
@@ -1089,529 +925,6 @@ int launch_rows(const GemmParams& p, int epi, int out_dt, bool has_bias, hipStre
     return has_bias ? launch_rows_t<1, true, false>(p, st) : launch_rows_t<1, false, false>(p, st);
 }
 
-// ---- half tiles (256 tokens x 128 channels) with three stages ----
-// The half-tile form runs a problem's last partial round and whole small problems (a 2048 x 3072 x 3072 linear is 96
-// full tiles, i.e. 192 half tiles on 192 CUs).  A half tile's k-step has half the MFMAs of a full one, and with two
-// stages its loads get about 1.25 k-steps to arrive: it waits on memory latency (about 1.1 us per k-step against
-// 0.55 us of MFMAs).  Its stage is 48 KiB (128 weight rows, then 256 token rows), so three fit the LDS when the
-// epilogue stores from registers instead of staging its tile: the loads of k-step g+3 go out during k-step g, one
-// barrier per k-step both frees stage g and publishes stage g+1, and the loads get about 1.9 k-steps.
-// Every output element goes through the same MFMA sequence and epilogue arithmetic as in the full tiles (weight row at
-// A-row n % 32, token at B-column m % 32, k ascending), so the output is bitwise the full-tile kernel's.
-// Each wave loads 32 weight rows and 64 token rows per k-step (12 LDS-DMA instructions) plus the two scale loads.
-constexpr int H3S_STAGE = (128 + 256) * ROWB;       // 48 KiB
-constexpr int H3S_A = 128 * ROWB;                   // token rows start after the 128 weight rows
-constexpr int H3S_NSTAGE = 3;
-constexpr int H3S_NSCALE = 4;                       // the cursor runs up to 3 tiles ahead (1 k-step per tile)
-constexpr int H3S_SCALES_OFF = H3S_NSTAGE * H3S_STAGE;
-constexpr int H3S_JUNK_OFF = H3S_SCALES_OFF + H3S_NSCALE * SCALE_SET;
-constexpr int H3S_LDS = H3S_JUNK_OFF + 512;
-static_assert(H3S_LDS <= 160 * 1024, "LDS of one CU");
-constexpr int H3S_LOADS = 14;                       // per wave and k-step: 4 weight + 8 token + 2 scale loads
-
-// Half-tile launch: workgroup id -> (tile position in the full-tile order, column half).  The full-tile launch before it
-// took workgroups b < full of the XCD-contiguous map over all T full tiles, i.e. the first full / 8 positions of each of
-// the 8 per-XCD ranges; the R = T - full positions left are the tails of those ranges.  They are listed range by range
-// (so consecutive entries are consecutive positions), split in two halves each, and dealt to the half-tile workgroups
-// by the same XCD-contiguous rule: the two halves of a tile and neighbouring tiles run on one XCD and share its L2.
-__device__ __forceinline__ void half_tile_of(const GemmParams& p, int id, int n_half, int& tm, int& tn) {
-    const int xcd = id & 7, local = id >> 3;
-    const int per = n_half >> 3, rem = n_half & 7;
-    const int lid = (xcd < rem) ? xcd * (per + 1) + local : rem * (per + 1) + (xcd - rem) * per + local;
-    int k = lid >> 1;
-    const int T = p.tiles_m * p.tiles_n, pT = T >> 3, rT = T & 7, done = p.half_first >> 3;
-    int c = 0;
-    for (; c < 7; ++c) {
-        const int n_c = pT + (c < rT ? 1 : 0) - done;
-        if (k < n_c) break;
-        k -= n_c;
-    }
-    const int pos = ((c < rT) ? c * (pT + 1) : rT * (pT + 1) + (c - rT) * pT) + done + k;
-    const int in_group = p.group_m * p.tiles_n;
-    const int g = pos / in_group;
-    const int first = g * p.group_m;
-    const int gsz = min(p.tiles_m - first, p.group_m);
-    const int r = pos - g * in_group;
-    tm = first + r % gsz;
-    tn = 2 * (r / gsz) + (lid & 1);
-}
-
-struct Half3Cursor {
-    v4u rw, ra, rsa, rsb;
-    uint32_t vw[2], va[2], vw_t[2], va_t[2];        // lane parts (even / odd 8-row groups); _t: the K-tail k-step
-    uint32_t row8_w, row8_a;
-    uint32_t sa_off, sb_off;
-    uint32_t dsa, dsb;                              // this wave's share of the tile's scale set (junk when unused)
-    int c, ks, nk;
-    bool valid;
-};
-
-__device__ __forceinline__ void h3s_cursor_set(Half3Cursor& I, const GroupedParams& gp, int c, uint32_t lds0,
-                                               int wave, int lane) {
-    const int id = (int)blockIdx.x + c * (int)gridDim.x;
-    I.c = c;
-    I.ks = 0;
-    I.valid = id < gp.total_tiles;
-    const uint32_t set = lds0 + H3S_SCALES_OFF + (uint32_t)(c % H3S_NSCALE) * SCALE_SET;
-    I.dsa = set + 256u * (uint32_t)wave;
-    I.dsb = wave < 2 ? set + 1024u + 256u * (uint32_t)wave : lds0 + H3S_JUNK_OFF;
-    if (!I.valid) {
-#pragma unroll
-        for (int e = 0; e < 2; ++e) I.vw[e] = I.va[e] = I.vw_t[e] = I.va_t[e] = OOB;
-        I.sa_off = I.sb_off = OOB;
-        I.nk = 1;
-        return;
-    }
-    int tm, tn;
-    const GemmParams& p = gp.g[0];
-    half_tile_of(p, id, gp.total_tiles, tm, tn);
-    I.nk = (p.K + BK - 1) / BK;
-    const uint32_t lrow = (uint32_t)(lane >> 3);
-    const uint32_t lch[2] = {(uint32_t)((lane & 7) ^ swz((int)lrow)), (uint32_t)((lane & 7) ^ swz((int)lrow + 8))};
-    const int64_t wrow0 = (int64_t)tn * (BN / 2) + 32 * wave;    // this wave's 32 weight rows
-    const int64_t arow0 = (int64_t)tm * BM + 64 * wave;          // ... and 64 token rows
-    I.rw = buffer_desc(p.w, p.w_bytes);
-    I.ra = buffer_desc(p.a, p.a_bytes);
-    const uint32_t ktail = (uint32_t)(p.K % BK);
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-        const uint32_t c16 = 16u * lch[e];
-        I.vw[e] = (wrow0 >= p.N) ? OOB : (uint32_t)((wrow0 + lrow) * p.ldw) + c16;   // rows past N: past the range
-        I.va[e] = (arow0 >= p.M) ? OOB : (uint32_t)((arow0 + lrow) * p.lda) + c16;   // rows past M: past the range
-        const bool cut = ktail != 0 && c16 >= ktail;
-        I.vw_t[e] = cut ? OOB : I.vw[e];
-        I.va_t[e] = cut ? OOB : I.va[e];
-    }
-    I.row8_w = (uint32_t)(8 * p.ldw);
-    I.row8_a = (uint32_t)(8 * p.lda);
-    I.rsa = buffer_desc(p.sa, p.sa_stride ? (uint32_t)((p.M - 1) * p.sa_stride * 4 + 4) : 4u);
-    I.rsb = buffer_desc(p.sb, p.sb_stride ? (uint32_t)((p.w_rows - 1) * p.sb_stride * 4 + 4) : 4u);
-    const int64_t srow = arow0 + lane;                            // sa of token row 64 wave + lane
-    I.sa_off = (srow < p.M) ? (uint32_t)(srow * p.sa_stride * 4) : OOB;
-    const int64_t wr = (int64_t)tn * (BN / 2) + 64 * wave + lane;  // waves 0, 1: sb of the tile's 128 weight rows
-    I.sb_off = (wave < 2 && wr < p.N) ? (uint32_t)(wr * p.sb_stride * 4) : OOB;
-}
-
-__device__ __forceinline__ void h3s_cursor_next(Half3Cursor& I, const GroupedParams& gp, uint32_t lds0, int wave,
-                                                int lane) {
-    if (++I.ks == I.nk) h3s_cursor_set(I, gp, I.c + 1, lds0, wave, lane);
-}
-
-// Load j (0..13) of the cursor's k-step into stage `st`: 0..3 the wave's weight rows (8 per instruction), 4..11 its
-// token rows, 12 / 13 the scales (into the tile's scale set at its first k-step, else into the scratch slot).
-__device__ __forceinline__ void h3s_issue_one(const Half3Cursor& I, uint32_t st, uint32_t lds0, int wave, int j) {
-    const bool last = I.ks == I.nk - 1;
-    const uint32_t k0 = (uint32_t)I.ks * BK;
-    if (j < 4) {
-        const uint32_t off = (last ? I.vw_t[j & 1] : I.vw[j & 1]);
-        dma16(I.rw, st + (uint32_t)(32 * wave + 8 * j) * ROWB, off == OOB ? OOB : off + k0 + (uint32_t)j * I.row8_w);
-    } else if (j < 12) {
-        const int i = j - 4;
-        const uint32_t off = (last ? I.va_t[i & 1] : I.va[i & 1]);
-        dma16(I.ra, st + H3S_A + (uint32_t)(64 * wave + 8 * i) * ROWB,
-              off == OOB ? OOB : off + k0 + (uint32_t)i * I.row8_a);
-    } else {
-        const bool real = I.valid && I.ks == 0;
-        if (j == 12) dma4(I.rsa, real ? I.dsa : lds0 + H3S_JUNK_OFF, real ? I.sa_off : OOB);
-        else dma4(I.rsb, real ? I.dsb : lds0 + H3S_JUNK_OFF, real ? I.sb_off : OOB);
-    }
-}
-
-// Fragment f of a sub-step (0, 1: the wave's two 32-row weight tiles; 2..5: its four 32-row token tiles).
-__device__ __forceinline__ void h3s_read(const uint8_t* stage, int wn, int wm, int lane, int sub, int f, v8i af[4],
-                                         v8i bf[4]) {
-    if (f < 2) af[f] = read_frag(stage + (wn * 64 + 32 * f) * ROWB, lane, sub);
-    else bf[f - 2] = read_frag(stage + H3S_A + (wm * 128 + 32 * (f - 2)) * ROWB, lane, sub);
-}
-
-// One k-step over 16 MFMA slots (u < 8 sub-step 0, u >= 8 sub-step 1):
-//   u < 6       the 6 sub-step-1 fragment reads of stage g;
-//   u == 7      lgkmcnt(0) + vmcnt(14) + barrier: every wave's reads of stage g have returned (it is free) and k-step
-//               g+1 has landed (only the loads of k-step g+2 may still be in flight);
-//   8 <= u < 15 the 14 loads of k-step g+3 into stage g, two per MFMA;
-//   8 <= u < 14 the 6 sub-step-0 fragment reads of k-step g+1.
-template <bool READ_NEXT>
-__device__ __forceinline__ void h3s_kstep(uint8_t* lds, uint32_t lds0, int s0, const Half3Cursor& I, int wave, int wn,
-                                          int wm, int lane, v16f acc[4][4], v8i fa0[4], v8i fb0[4], v8i fa1[4],
-                                          v8i fb1[4]) {
-    const int s1 = s0 == H3S_NSTAGE - 1 ? 0 : s0 + 1;
-    const uint8_t* cur = lds + s0 * H3S_STAGE;
-    const uint8_t* nxt = lds + s1 * H3S_STAGE;
-    const uint32_t st = lds0 + (uint32_t)s0 * H3S_STAGE;
-    constexpr int NEXT_ORDER[6] = {0, 2, 3, 4, 5, 1};   // weight tile 0 and the token tiles first: MFMA t uses
-                                                        // weight tile t / 4 and token tile t % 4
-#pragma unroll
-    for (int u = 0; u < 16; ++u) {
-        if (u < 8) mfma_one(acc, fa0, fb0, u);
-        else mfma_one(acc, fa1, fb1, u - 8);
-        if (u < 6) h3s_read(cur, wn, wm, lane, 1, u, fa1, fb1);
-        if (u == 7) {
-            wait_lgkm0();
-            __builtin_amdgcn_s_waitcnt(vmcnt_imm(H3S_LOADS));
-            barrier_nofence();
-        }
-        if (u >= 8 && u < 15) {
-            h3s_issue_one(I, st, lds0, wave, 2 * (u - 8));
-            h3s_issue_one(I, st, lds0, wave, 2 * (u - 8) + 1);
-        }
-        if (READ_NEXT && u >= 8 && u < 14) h3s_read(nxt, wn, wm, lane, 0, NEXT_ORDER[u - 8], fa0, fb0);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-}
-
-// Epilogue of a wave's NI x NJ MFMA blocks from the accumulators: register 4q + r of block (i, j) is channel
-// col0 + 32 i + 8 q + 4 (lane >> 5) + r of token mrow0 + 32 j + (lane & 31); sa_l[sa0 + t] and sb_l[sb0 + c] (LDS)
-// hold the scales of token mrow0 + t and channel col0 + c.  Without staging each lane stores its 4 consecutive
-// channels (8 bytes, 16 contiguous bytes with the partner lane l ^ 32), so a store instruction touches 32 rows.
-// STAGED (bf16 / fp16 outputs): the 32 tokens of block row j go through the wave's LDS area `stg` (rows of NI x 64
-// bytes at a stride padded by 16 bytes) and come back as 16-byte chunks, chunk c of row t at lane (32 t + c) % 64 of
-// instruction (32 t + c) / 64 -- every store then writes whole row segments of NI x 64 bytes (the store path handles
-// about one 128-byte line per cycle, so the lines an instruction touches are what it costs).  Rows past M fall
-// outside the output descriptor's range, columns past N get an out-of-range offset.
-template <int OUT_DT, bool HAS_BIAS, int EPI, int NI, int NJ, int AI, int AJ, bool STAGED = false>
-__device__ __forceinline__ void reg_epilogue(const GemmParams& p, int col0, int mrow0, const float* sa_l, int sa0,
-                                             const float* sb_l, int sb0, int lane, v16f (&acc)[AI][AJ],
-                                             uint8_t* stg = nullptr) {
-    constexpr int CH = NI * 4;                          // 16-byte chunks per staged token row
-    constexpr int RS = CH * 16 + 16;                    // staged row stride (padded: rows fall on other banks)
-    static_assert(!STAGED || (32 * CH) % 64 == 0, "whole store instructions per block row");
-    static_assert(NI <= AI && NJ <= AJ, "blocks of the accumulator array");
-    const int hi = lane >> 5, mj = lane & 31;
-    if (OUT_DT == H3FP8_DT_F32) {
-        float* yf = reinterpret_cast<float*>(p.y);
-#pragma unroll
-        for (int i = 0; i < NI; ++i)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int j = 0; j < NJ; ++j) {
-                    const int n = col0 + 32 * i + 8 * q + 4 * hi;
-                    const int m = mrow0 + 32 * j + mj;
-                    if (n < p.N && m < p.M) {
-                        const v4f v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
-                                       acc[i][j][4 * q + 3]};
-                        *reinterpret_cast<v4f*>(yf + (int64_t)m * p.ldy + n) = v;
-                    }
-                }
-        return;
-    }
-    const __amdgpu_buffer_rsrc_t yr = make_rsrc(p.y, p.y_bytes);
-    const uint32_t row2 = (uint32_t)p.ldy * 2u;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        const int m = mrow0 + 32 * j + mj;
-        const float sam = sa_l[sa0 + 32 * j + mj];
-        uint32_t rmax = 0;
-        if (STAGED) wave_sync();                        // the previous block row's reads before these writes
-#pragma unroll
-        for (int i = 0; i < NI; ++i)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int n = col0 + 32 * i + 8 * q + 4 * hi;
-                const v4f sbn = *reinterpret_cast<const v4f*>(sb_l + sb0 + 32 * i + 8 * q + 4 * hi);
-                float bn[4] = {0, 0, 0, 0};
-                if (HAS_BIAS) {
-                    const int nc = n < p.N ? n : 0;
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) bn[r] = load_bias(p.bias, nc + r, OUT_DT);
-                }
-                float v[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float t = sbn[r] * acc[i][j][4 * q + r];
-                    v[r] = HAS_BIAS ? __builtin_fmaf(sam, t, bn[r]) : sam * t;
-                }
-                uint32_t lo, hi2;
-                if (OUT_DT) {
-                    lo = fp16_rne(v[0]) | (fp16_rne(v[1]) << 16);
-                    hi2 = fp16_rne(v[2]) | (fp16_rne(v[3]) << 16);
-                } else {
-                    lo = cvt_bf16x2(v[0], v[1]);
-                    hi2 = cvt_bf16x2(v[2], v[3]);
-                }
-                if (EPI == EPI_AMAX && n < p.N && m < p.M)
-                    rmax = OUT_DT ? max_abs_f16x2(max_abs_f16x2(rmax, lo), hi2)
-                                  : max_abs_bf16x2(max_abs_bf16x2(rmax, lo), hi2);
-                const v2u32 val = {lo, hi2};
-                if (STAGED) {
-                    *reinterpret_cast<v2u32*>(stg + mj * RS + (4 * i + q) * 16 + 8 * hi) = val;
-                } else {
-                    const uint32_t off = (n < p.N) ? (uint32_t)m * row2 + (uint32_t)n * 2u : OOB;
-                    __builtin_amdgcn_raw_buffer_store_b64(val, yr, off, 0, 0);
-                }
-            }
-        if (STAGED) {
-            wave_sync();                                // every lane's writes before any lane's reads
-            constexpr int NS = 32 * CH / 64;
-            v4u v[NS];
-            uint32_t off[NS];
-#pragma unroll
-            for (int s2 = 0; s2 < NS; ++s2) {           // all reads before the first store
-                const int idx = 64 * s2 + lane, t = idx / CH, c = idx - t * CH;
-                v[s2] = *reinterpret_cast<const v4u*>(stg + t * RS + c * 16);
-                const int n = col0 + 8 * c;
-                off[s2] = (n < p.N) ? (uint32_t)(mrow0 + 32 * j + t) * row2 + (uint32_t)n * 2u : OOB;
-            }
-#pragma unroll
-            for (int s2 = 0; s2 < NS; ++s2) __builtin_amdgcn_raw_buffer_store_b128(v[s2], yr, off[s2], 0, 0);
-        }
-        if (EPI == EPI_AMAX) {
-            const uint32_t o = (uint32_t)__shfl_xor((int)rmax, 32, 64);
-            rmax = rmax > o ? rmax : o;
-            if (hi == 0 && m < p.M && rmax) atomicMax(reinterpret_cast<unsigned int*>(p.row_amax) + m, rmax);
-        }
-    }
-}
-
-// A half tile's wave owns 2 x 4 blocks: channels tn * 128 + 64 wn onwards, tokens tm * 256 + 128 wm onwards.
-template <int OUT_DT, bool HAS_BIAS, int EPI>
-__device__ __forceinline__ void h3s_epilogue(const GemmParams& p, int tm, int tn, const uint8_t* lds, int set, int wn,
-                                             int wm, int lane, v16f (&acc)[4][4]) {
-    const float* sa_l = reinterpret_cast<const float*>(lds + H3S_SCALES_OFF + set * SCALE_SET);
-    const float* sb_l = sa_l + 256;
-    reg_epilogue<OUT_DT, HAS_BIAS, EPI, 2, 4>(p, tn * (BN / 2) + wn * 64, tm * BM + wm * 128, sa_l, wm * 128, sb_l,
-                                              wn * 64, lane, acc);
-}
-
-template <int OUT_DT, bool HAS_BIAS, int EPI>
-__global__ void __launch_bounds__(256, 1) gemm_half3_kernel(GroupedParams gp) {
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[H3S_LDS];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int wn = wave & 1, wm = wave >> 1;
-    const int G = (int)gridDim.x;
-    const uint32_t lds0 = lds_addr(lds);
-    Half3Cursor I;
-    h3s_cursor_set(I, gp, 0, lds0, wave, lane);
-    if (!I.valid) return;
-    // prologue: k-steps 0, 1, 2 in flight (14 loads each), then stage 0 published
-#pragma unroll
-    for (int s = 0; s < H3S_NSTAGE; ++s) {
-#pragma unroll
-        for (int j = 0; j < H3S_LOADS; ++j) h3s_issue_one(I, lds0 + (uint32_t)s * H3S_STAGE, lds0, wave, j);
-        if (I.valid) h3s_cursor_next(I, gp, lds0, wave, lane);
-    }
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * H3S_LOADS));
-    barrier_nofence();
-    v8i fa0[4], fb0[4], fa1[4], fb1[4];
-#pragma unroll
-    for (int f = 0; f < 6; ++f) h3s_read(lds, wn, wm, lane, 0, f, fa0, fb0);
-    int s0 = 0;
-    for (int c = 0;; ++c) {
-        const int id = (int)blockIdx.x + c * G;
-        int tm, tn;
-        const GemmParams& p = gp.g[0];
-        half_tile_of(p, id, gp.total_tiles, tm, tn);
-        const int nk = (p.K + BK - 1) / BK;
-        v16f acc[4][4];                                 // acc[0..1][*] used
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-        for (int ks = 0; ks < nk - 1; ++ks) {
-            h3s_kstep<true>(lds, lds0, s0, I, wave, wn, wm, lane, acc, fa0, fb0, fa1, fb1);
-            if (I.valid) h3s_cursor_next(I, gp, lds0, wave, lane);
-            s0 = s0 == H3S_NSTAGE - 1 ? 0 : s0 + 1;
-        }
-        h3s_kstep<false>(lds, lds0, s0, I, wave, wn, wm, lane, acc, fa0, fb0, fa1, fb1);
-        if (I.valid) h3s_cursor_next(I, gp, lds0, wave, lane);
-        s0 = s0 == H3S_NSTAGE - 1 ? 0 : s0 + 1;
-        h3s_epilogue<OUT_DT, HAS_BIAS, EPI>(p, tm, tn, lds, c % H3S_NSCALE, wn, wm, lane, acc);
-        __builtin_amdgcn_sched_barrier(0);
-        if (id + G >= gp.total_tiles) break;
-#pragma unroll
-        for (int f = 0; f < 6; ++f) h3s_read(lds + s0 * H3S_STAGE, wn, wm, lane, 0, f, fa0, fb0);
-    }
-    wait_vm0();                                         // the trailing zero-fill loads have landed before the exit
-}
-
-// ---- 128 x 192 tiles, one per workgroup (problems that fit one round) ----
-// A problem whose 256 x 256 tiles number at most half the CUs runs as half tiles, which can still leave CUs idle: the
-// single linear 2048 x 3072 x 3072 has 96 full tiles, 192 half tiles, on 256 CUs.  Tiles of 128 token rows x 192
-// weight rows cover it with 16 x 16 = 256 workgroups, one per CU, each loading 40 KiB per k-step (half tiles: 48).
-// The four waves own 96 weight rows x 64 token rows each (3 x 2 MFMA blocks).  Every output element gets the same
-// MFMA sequence as in the other forms (k sub-steps of 64 in order from a zero accumulator), so the same bits.
-constexpr int W192_WR = 192;                            // weight rows per tile
-constexpr int W192_TR = 128;                            // token rows per tile
-constexpr int W192_STAGE = (W192_WR + W192_TR) * ROWB;  // 40 KiB
-constexpr int W192_A = W192_WR * ROWB;                  // token rows start after the weight rows
-constexpr int W192_NSTAGE = 3;
-constexpr int W192_SCALES_OFF = W192_NSTAGE * W192_STAGE;
-constexpr int W192_JUNK_OFF = W192_SCALES_OFF + SCALE_SET;
-constexpr int W192_STG_OFF = W192_JUNK_OFF + 512;      // the epilogue's staging: per wave 32 rows of 192 + 16 bytes
-constexpr int W192_STG_PER_WAVE = 32 * (3 * 64 + 16);
-constexpr int W192_LDS = W192_STG_OFF + 4 * W192_STG_PER_WAVE;
-static_assert(W192_LDS <= 160 * 1024, "LDS of one CU");
-constexpr int W192_LOADS = 12;                          // per wave and k-step: 6 weight + 4 token + 2 scale loads
-constexpr int W192_GROUP_M = 8;                         // token-tile rows per group of the XCD-contiguous tile map
-                                                        // (c1: an XCD's 32 tiles read 5.5 MB of operands, with 4 rows
-                                                        // 6.3 MB; measured 1-3 % faster than 4)
-
-struct W192Loader {
-    v4u rw, ra, rsa, rsb;
-    uint32_t vw[2], va[2], vw_t[2], va_t[2];            // lane parts (even / odd 8-row groups); _t: the K-tail k-step
-    uint32_t row8_w, row8_a;
-    uint32_t sa_off, sb_off;
-    uint32_t dsa, dsb;                                  // this wave's share of the tile's scale set (junk when unused)
-    int wgroups, agroups;                               // this wave's 8-row groups that start inside N / M
-    int nk;
-};
-
-// Wave w loads weight rows 48 w .. 48 w + 47 and token rows 32 w .. 32 w + 31 of the tile (6 and 4 groups of 8 rows);
-// waves 0, 1 the sa of the tile's 128 token rows, waves 0..2 the sb of its 192 weight rows.
-__device__ __forceinline__ void w192_loader_set(W192Loader& L, const GemmParams& p, int tm, int tn, uint32_t lds0,
-                                                int wave, int lane) {
-    L.nk = (p.K + BK - 1) / BK;
-    const uint32_t lrow = (uint32_t)(lane >> 3);
-    const uint32_t lch[2] = {(uint32_t)((lane & 7) ^ swz((int)lrow)), (uint32_t)((lane & 7) ^ swz((int)lrow + 8))};
-    const int64_t wrow0 = (int64_t)tn * W192_WR + 48 * wave;
-    const int64_t arow0 = (int64_t)tm * W192_TR + 32 * wave;
-    const int64_t wg = wrow0 < p.N ? (p.N - wrow0 + 7) / 8 : 0, ag = arow0 < p.M ? (p.M - arow0 + 7) / 8 : 0;
-    L.wgroups = (int)(wg < 6 ? wg : 6);
-    L.agroups = (int)(ag < 4 ? ag : 4);
-    L.rw = buffer_desc(p.w, p.w_bytes);
-    L.ra = buffer_desc(p.a, p.a_bytes);
-    const uint32_t ktail = (uint32_t)(p.K % BK);
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-        const uint32_t c16 = 16u * lch[e];
-        L.vw[e] = L.wgroups ? (uint32_t)((wrow0 + lrow) * p.ldw) + c16 : OOB;
-        L.va[e] = L.agroups ? (uint32_t)((arow0 + lrow) * p.lda) + c16 : OOB;
-        const bool cut = ktail != 0 && c16 >= ktail;
-        L.vw_t[e] = cut ? OOB : L.vw[e];
-        L.va_t[e] = cut ? OOB : L.va[e];
-    }
-    L.row8_w = (uint32_t)(8 * p.ldw);
-    L.row8_a = (uint32_t)(8 * p.lda);
-    L.rsa = buffer_desc(p.sa, p.sa_stride ? (uint32_t)((p.M - 1) * p.sa_stride * 4 + 4) : 4u);
-    L.rsb = buffer_desc(p.sb, p.sb_stride ? (uint32_t)((p.w_rows - 1) * p.sb_stride * 4 + 4) : 4u);
-    const uint32_t set = lds0 + W192_SCALES_OFF;
-    L.dsa = wave < 2 ? set + 256u * (uint32_t)wave : lds0 + W192_JUNK_OFF;
-    L.dsb = wave < 3 ? set + 1024u + 256u * (uint32_t)wave : lds0 + W192_JUNK_OFF;
-    const int64_t srow = (int64_t)tm * W192_TR + 64 * wave + lane;
-    L.sa_off = (wave < 2 && srow < p.M) ? (uint32_t)(srow * p.sa_stride * 4) : OOB;
-    const int64_t wr = (int64_t)tn * W192_WR + 64 * wave + lane;
-    L.sb_off = (wave < 3 && wr < p.N) ? (uint32_t)(wr * p.sb_stride * 4) : OOB;
-}
-
-// Load j (0..11) of k-step kl into stage `st`: 0..5 the wave's weight rows (8 per instruction), 6..9 its token rows,
-// 10 / 11 the scales (into the scale set at k-step 0, else into the scratch slot).  K-steps past the last one load
-// zeros (every k-step issues the same 12 loads, which the vmcnt waits count on).
-__device__ __forceinline__ void w192_issue_one(const W192Loader& L, int kl, uint32_t st, uint32_t lds0, int wave,
-                                               int j) {
-    const bool live = kl < L.nk;
-    const bool last = kl == L.nk - 1;
-    const uint32_t k0 = (uint32_t)kl * BK;
-    if (j < 6) {
-        const uint32_t off = last ? L.vw_t[j & 1] : L.vw[j & 1];
-        const bool ok = live && j < L.wgroups && off != OOB;
-        dma16(L.rw, st + (uint32_t)(48 * wave + 8 * j) * ROWB, ok ? off + k0 + (uint32_t)j * L.row8_w : OOB);
-    } else if (j < 10) {
-        const int i = j - 6;
-        const uint32_t off = last ? L.va_t[i & 1] : L.va[i & 1];
-        const bool ok = live && i < L.agroups && off != OOB;
-        dma16(L.ra, st + W192_A + (uint32_t)(32 * wave + 8 * i) * ROWB, ok ? off + k0 + (uint32_t)i * L.row8_a : OOB);
-    } else {
-        const bool real = kl == 0;
-        if (j == 10) dma4(L.rsa, real ? L.dsa : lds0 + W192_JUNK_OFF, real ? L.sa_off : OOB);
-        else dma4(L.rsb, real ? L.dsb : lds0 + W192_JUNK_OFF, real ? L.sb_off : OOB);
-    }
-}
-
-// Fragment f of a sub-step (0..2: the wave's three 32-row weight blocks; 3, 4: its two 32-row token blocks).
-__device__ __forceinline__ void w192_read(const uint8_t* stage, int wn, int wm, int lane, int sub, int f, v8i af[3],
-                                          v8i bf[2]) {
-    if (f < 3) af[f] = read_frag(stage + (wn * 96 + 32 * f) * ROWB, lane, sub);
-    else bf[f - 3] = read_frag(stage + W192_A + (wm * 64 + 32 * (f - 3)) * ROWB, lane, sub);
-}
-
-__device__ __forceinline__ void w192_mfma(v16f acc[3][2], const v8i af[3], const v8i bf[2], int t) {
-    acc[t >> 1][t & 1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af[t >> 1], bf[t & 1], acc[t >> 1][t & 1], 0, 0,
-                                                                         0, 0, 0, 0);
-}
-
-// K-step ks over 12 MFMA slots (u < 6 sub-step 0, u >= 6 sub-step 1):
-//   u < 5        the 5 sub-step-1 fragment reads of stage ks;
-//   u == 5       lgkmcnt(0) + vmcnt(12) + barrier: every wave's reads of stage ks have returned (it is free) and k-step
-//                ks + 1 has landed (only the loads of k-step ks + 2 may still be in flight);
-//   6 <= u < 12  the 12 loads of k-step ks + 3 into stage ks, two per MFMA;
-//   6 <= u < 11  the 5 sub-step-0 fragment reads of k-step ks + 1.
-template <bool READ_NEXT>
-__device__ __forceinline__ void w192_kstep(uint8_t* lds, uint32_t lds0, int s0, int ks, const W192Loader& L, int wave,
-                                           int wn, int wm, int lane, v16f acc[3][2], v8i fa0[3], v8i fb0[2],
-                                           v8i fa1[3], v8i fb1[2]) {
-    const int s1 = s0 == W192_NSTAGE - 1 ? 0 : s0 + 1;
-    const uint8_t* cur = lds + s0 * W192_STAGE;
-    const uint8_t* nxt = lds + s1 * W192_STAGE;
-    const uint32_t st = lds0 + (uint32_t)s0 * W192_STAGE;
-    constexpr int NEXT_ORDER[5] = {0, 3, 4, 1, 2};      // weight block 0 and the token blocks first: MFMA t uses
-                                                        // weight block t / 2 and token block t % 2
-#pragma unroll
-    for (int u = 0; u < 12; ++u) {
-        if (u < 6) w192_mfma(acc, fa0, fb0, u);
-        else w192_mfma(acc, fa1, fb1, u - 6);
-        if (u < 5) w192_read(cur, wn, wm, lane, 1, u, fa1, fb1);
-        if (u == 5) {
-            wait_lgkm0();
-            __builtin_amdgcn_s_waitcnt(vmcnt_imm(W192_LOADS));
-            barrier_nofence();
-        }
-        if (u >= 6) {
-            w192_issue_one(L, ks + 3, st, lds0, wave, 2 * (u - 6));
-            w192_issue_one(L, ks + 3, st, lds0, wave, 2 * (u - 6) + 1);
-        }
-        if (READ_NEXT && u >= 6 && u < 11) w192_read(nxt, wn, wm, lane, 0, NEXT_ORDER[u - 6], fa0, fb0);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-}
-
-// One tile per workgroup: the launch has exactly as many workgroups as tiles, all resident at once (at most one per
-// CU), so there is no persistent loop.
-template <int OUT_DT, bool HAS_BIAS, int EPI>
-__global__ void __launch_bounds__(256, 1) gemm_w192_kernel(GemmParams p) {
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[W192_LDS];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int wn = wave & 1, wm = wave >> 1;
-    const uint32_t lds0 = lds_addr(lds);
-    const int tiles_m = (p.M + W192_TR - 1) / W192_TR, tiles_n = (p.N + W192_WR - 1) / W192_WR;
-    int tm, tn;
-    tile_of((int)blockIdx.x, tiles_m * tiles_n, tiles_m, tiles_n, W192_GROUP_M, tm, tn);
-    W192Loader L;
-    w192_loader_set(L, p, tm, tn, lds0, wave, lane);
-    // prologue: k-steps 0, 1, 2 in flight (12 loads each), then stage 0 published
-#pragma unroll
-    for (int s = 0; s < W192_NSTAGE; ++s) {
-#pragma unroll
-        for (int j = 0; j < W192_LOADS; ++j) w192_issue_one(L, s, lds0 + (uint32_t)s * W192_STAGE, lds0, wave, j);
-    }
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * W192_LOADS));
-    barrier_nofence();
-    v8i fa0[3], fb0[2], fa1[3], fb1[2];
-#pragma unroll
-    for (int f = 0; f < 5; ++f) w192_read(lds, wn, wm, lane, 0, f, fa0, fb0);
-    v16f acc[3][2];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-    int s0 = 0;
-    for (int ks = 0; ks < L.nk - 1; ++ks) {
-        w192_kstep<true>(lds, lds0, s0, ks, L, wave, wn, wm, lane, acc, fa0, fb0, fa1, fb1);
-        s0 = s0 == W192_NSTAGE - 1 ? 0 : s0 + 1;
-    }
-    w192_kstep<false>(lds, lds0, s0, L.nk - 1, L, wave, wn, wm, lane, acc, fa0, fb0, fa1, fb1);
-    const float* sa_l = reinterpret_cast<const float*>(lds + W192_SCALES_OFF);
-    reg_epilogue<OUT_DT, HAS_BIAS, EPI, 3, 2, 3, 2, true>(p, tn * W192_WR + wn * 96, tm * W192_TR + wm * 64, sa_l,
-                                                          wm * 64, sa_l + 256, wn * 96, lane, acc,
-                                                          lds + W192_STG_OFF + wave * W192_STG_PER_WAVE);
-    wait_vm0();                                         // the trailing zero-fill loads have landed before the exit
-}
-
 __global__ void __launch_bounds__(256) fill_zero_kernel(float* p, int64_t n) {
     int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i < n) p[i] = 0.0f;
@@ -1644,76 +957,35 @@ int dispatch(const GroupedParams& gp, int out_dt, bool has_bias, hipStream_t st)
     return has_bias ? launch_one<1, true, EPI, false>(gp, st) : launch_one<1, false, EPI, false>(gp, st);
 }
 
-template <int OUT_DT, bool HAS_BIAS, int EPI>
-int launch_half3(const GroupedParams& gp, hipStream_t st) {
-    hipLaunchKernelGGL((gemm_half3_kernel<OUT_DT, HAS_BIAS, EPI>), dim3(grid_for(gp.total_tiles)), dim3(256), 0, st, gp);
-    H3_CHECK_HIP(hipGetLastError());
-    return H3FP8_OK;
-}
-
-int dispatch_half3(const GroupedParams& gp, int epi, int out_dt, bool has_bias, hipStream_t st) {
-    if (out_dt == H3FP8_DT_F32) return launch_half3<H3FP8_DT_F32, false, EPI_PLAIN>(gp, st);
-    if (epi == EPI_AMAX) {
-        if (out_dt == H3FP8_DT_BF16)
-            return has_bias ? launch_half3<0, true, EPI_AMAX>(gp, st) : launch_half3<0, false, EPI_AMAX>(gp, st);
-        return has_bias ? launch_half3<1, true, EPI_AMAX>(gp, st) : launch_half3<1, false, EPI_AMAX>(gp, st);
-    }
-    if (out_dt == H3FP8_DT_BF16)
-        return has_bias ? launch_half3<0, true, EPI_PLAIN>(gp, st) : launch_half3<0, false, EPI_PLAIN>(gp, st);
-    return has_bias ? launch_half3<1, true, EPI_PLAIN>(gp, st) : launch_half3<1, false, EPI_PLAIN>(gp, st);
-}
-
-template <int OUT_DT, bool HAS_BIAS, int EPI>
-int launch_w192(const GemmParams& p, int tiles, hipStream_t st) {
-    hipLaunchKernelGGL((gemm_w192_kernel<OUT_DT, HAS_BIAS, EPI>), dim3(tiles), dim3(256), 0, st, p);
-    H3_CHECK_HIP(hipGetLastError());
-    return H3FP8_OK;
-}
-
-int dispatch_w192(const GemmParams& p, int tiles, int epi, int out_dt, bool has_bias, hipStream_t st) {
-    if (out_dt == H3FP8_DT_F32) return launch_w192<H3FP8_DT_F32, false, EPI_PLAIN>(p, tiles, st);
-    if (epi == EPI_AMAX) {
-        if (out_dt == H3FP8_DT_BF16)
-            return has_bias ? launch_w192<0, true, EPI_AMAX>(p, tiles, st) : launch_w192<0, false, EPI_AMAX>(p, tiles, st);
-        return has_bias ? launch_w192<1, true, EPI_AMAX>(p, tiles, st) : launch_w192<1, false, EPI_AMAX>(p, tiles, st);
-    }
-    if (out_dt == H3FP8_DT_BF16)
-        return has_bias ? launch_w192<0, true, EPI_PLAIN>(p, tiles, st) : launch_w192<0, false, EPI_PLAIN>(p, tiles, st);
-    return has_bias ? launch_w192<1, true, EPI_PLAIN>(p, tiles, st) : launch_w192<1, false, EPI_PLAIN>(p, tiles, st);
-}
-
-// The last, partial round of a launch with full tiles leaves most CUs idle.  When its tiles fit one round as half
-// tiles (256 tokens x 128 channels, the same MFMAs per output element, so the same bits), the full-tile launch stops
-// at the last whole round and a half-tile launch covers the rest: a problem of T full tiles on G CUs runs
-// floor(T / G) full rounds and, if T mod G <= G / 2, the remainder as 2 (T mod G) half tiles.  Kernel 3 (SwiGLU pairs
-// gate and up rows inside a tile) always runs full tiles.  A problem that runs as half tiles alone takes 128 x 192
-// tiles instead when they occupy more CUs and still fit one round (gemm_w192_kernel).
+// Which tiles a problem of T 256 x 256 tiles on G CUs runs in (all forms give the same bits):
+//   * one of the smaller forms (gemm_tile.hip) when its tiles fit one round: the smallest that does, since a round lasts
+//     as long as one tile.  That includes every T <= G / 2 (256 x 128 tiles), and problems of up to G full tiles whose
+//     token rows are mostly padding (M = 320 is 2 x 256 rows but 3 x 128; 320 x 21 504 x 5376: 58.0 -> 44.1 us).
+//   * else full tiles in whole rounds, the last partial round cut into smaller tiles if at most half the CUs have one
+//     (T mod G <= G / 2); a fuller last round runs as full tiles.  Against a tail of four-wave 256 x 128 tiles:
+//     4100 x 5376 x 14336 255.0 -> 242.6 us (101 tiles left), 16 740 x 9216 x 3072 372.7 -> 364.1 (72 left).
+// Kernel 3 (SwiGLU pairs gate and up rows inside a tile) always runs full tiles.
 int launch_split(GroupedParams gp, int epi, int out_dt, bool has_bias, hipStream_t st) {
-    const int T = gp.g[0].tiles_m * gp.g[0].tiles_n;
+    const GemmParams& p = gp.g[0];
+    const int T = p.tiles_m * p.tiles_n;
     const int G = h3host::cu_count();
-    const int full = (epi == EPI_SWIGLU) ? T : (T / G) * G;
+    if (epi == EPI_SWIGLU) {
+        gp.total_tiles = T;
+        return dispatch<EPI_SWIGLU>(gp, H3FP8_DT_BF16, has_bias, st);
+    }
+    const int form = tile_form_for(p.M, p.N, G);
+    if (form < TILE_FORMS) return launch_tiles(p, form, out_dt, st);
+    const int full = (T / G) * G;
     const int rest = T - full;
-    // half_tile_of takes the full-tile launch to have covered the first full / 8 positions of each per-XCD range,
-    // which holds when full is a multiple of 8 (a CU count that is a multiple of 8, as on gfx950); otherwise the
-    // launch keeps full tiles throughout
-    const bool half = rest > 0 && 2 * rest <= G && full % 8 == 0;
-    const int full_tiles = half ? full : T;
-    if (full_tiles == 0) {
-        const GemmParams& p = gp.g[0];
-        const int64_t w192 = (int64_t)((p.M + W192_TR - 1) / W192_TR) * ((p.N + W192_WR - 1) / W192_WR);
-        if (w192 <= G && w192 > 2 * (int64_t)rest) return dispatch_w192(p, (int)w192, epi, out_dt, has_bias, st);
-    }
-    int rc = H3FP8_OK;
-    if (full_tiles > 0) {
-        gp.total_tiles = full_tiles;
-        if (epi == EPI_PLAIN) rc = dispatch<EPI_PLAIN>(gp, out_dt, has_bias, st);
-        else if (epi == EPI_AMAX) rc = dispatch<EPI_AMAX>(gp, out_dt, has_bias, st);
-        else rc = dispatch<EPI_SWIGLU>(gp, H3FP8_DT_BF16, has_bias, st);
-        if (rc || !half) return rc;
-    }
-    gp.g[0].half_first = full_tiles;
-    gp.total_tiles = 2 * rest;
-    return dispatch_half3(gp, epi, out_dt, has_bias, st);
+    // the tail's tile map takes the full-tile launch to have covered the first full / 8 positions of each per-XCD range,
+    // which holds when full is a multiple of 8 (a CU count that is a multiple of 8, as on gfx950); otherwise the launch
+    // keeps full tiles throughout
+    const bool tail = rest > 0 && 2 * rest <= G && full % 8 == 0;
+    gp.total_tiles = tail ? full : T;
+    const int rc = epi == EPI_PLAIN ? dispatch<EPI_PLAIN>(gp, out_dt, has_bias, st)
+                                    : dispatch<EPI_AMAX>(gp, out_dt, has_bias, st);
+    if (rc || !tail) return rc;
+    return launch_tile_tail(p, full, rest, G, out_dt, st);
 }
 
 constexpr int64_t kMaxBufferBytes = 0x7fff0000LL;   // buffer offsets are 32-bit; keep clear of the OOB marker

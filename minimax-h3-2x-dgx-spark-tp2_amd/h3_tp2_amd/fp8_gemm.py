@@ -184,9 +184,9 @@ def make_scaled_mm(orig):  # noqa: ANN001,ANN201
     return _mm
 
 
-# Install-check cases: (kind, M, N, K).  The small ones run as half tiles or 128 x 192 tiles and pin the edges; the
+# Install-check cases: (kind, M, N, K).  The small ones run as smaller tiles and pin the edges; the
 # 4100-row ones are the serving shapes the reference checks at install (h3_tp2/fp8_cutlass.py:211-213) -- 17 token tiles
-# x 21 weight tiles = 357 tiles, so they run the persistent full-tile kernel on every CU and its half-tile tail.
+# x 21 weight tiles = 357 tiles, so they run the persistent full-tile kernel on every CU and its tail of smaller tiles.
 SELFCHECK_CASES = (("int", 200, 400, 512), ("int", 333, 272, 1024), ("int", 129, 528, 3072),
                    ("int", 4100, 5376, 1024), ("rand", 200, 1040, 2048), ("rand", 4100, 5376, 7168),
                    ("rand", 4100, 21504, 5376))

@@ -1,0 +1,86 @@
+"""The smaller tiles of kernel 2 (one tile per workgroup; 32 x 64 ... 256 x 128 weight rows x token rows) and the last
+rounds cut into them.
+
+Each case's sizes take one form on 256 CUs (asserted from the tile counts), with ragged edges in M and N, K tails and one
+to five k-steps (the ring is deeper than the problem, or its parity differs).  Bits: equal to the grouped launch, which
+always runs 256 x 256 tiles, on random operands, where the MFMA's inexact accumulation would expose any change of order;
+integer operands are exact against the oracle, with sentinels around the output.
+"""
+import numpy as np
+import pytest
+import torch
+
+from _util import bits16, f32, int_operands, ref_gemm, serving_like
+
+pytestmark = pytest.mark.gpu
+
+FORMS = ((32, 64), (64, 64), (96, 64), (128, 64), (128, 128), (192, 128), (256, 128))
+# the form (index of FORMS), then M, N, K
+WHOLE = [(0, 33, 16, 16), (0, 65, 528, 1040), (1, 260, 1840, 272), (2, 500, 2320, 400), (3, 700, 2320, 144),
+         (4, 1000, 3008, 96), (5, 2040, 2992, 640), (6, 2300, 3312, 192), (6, 320, 21504, 256)]
+# last rounds: the form of the pieces, then M, N, K (264, 266, 286, 316, 356 full tiles)
+TAILS = [(0, 8300, 2032, 160), (1, 3400, 4800, 64), (3, 5600, 3200, 272), (4, 20200, 912, 128), (6, 22600, 1008, 400)]
+
+
+def _count(form, M, N):
+    tw, tt = FORMS[form]
+    return -(-M // tt) * -(-N // tw)
+
+
+def _takes(form, M, N, tail):
+    G = torch.cuda.get_device_properties(0).multi_processor_count
+    if not tail:
+        return min((f for f in range(len(FORMS)) if _count(f, M, N) <= G), default=None) == form
+    rest = -(-M // 256) * -(-N // 256) % G
+    pieces = [(f, 256 // tw * (256 // tt)) for f, (tw, tt) in enumerate(FORMS) if 256 % tw == 0]
+    return 0 < 2 * rest <= G and min(f for f, p in pieces if rest * p <= G) == form
+
+
+CASES = [(*c, False) for c in WHOLE] + [(*c, True) for c in TAILS]
+
+
+@pytest.mark.parametrize("form,M,N,K,tail", CASES)
+def test_form_equals_full_tiles(cuda, form, M, N, K, tail):
+    from h3_tp2_amd import ops
+    assert _takes(form, M, N, tail)
+    a, w, sa, sb = serving_like(M, N, K, seed=M + K, device=cuda)
+    y = ops.gemm(a, w, sa, sb)
+    (ref,) = ops.grouped_gemm([(a, w, sa, sb)])
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("form,M,N,K,tail", CASES)
+def test_form_integer_exact_with_guards(cuda, form, M, N, K, tail):
+    from h3_tp2_amd import ops
+    a, w, sa, sb = int_operands(M, N, K, seed=M + N, device=cuda)
+    guard = 4096
+    buf = torch.full((M * N + 2 * guard,), float("nan"), device=cuda, dtype=torch.bfloat16)
+    buf[:guard] = 7.0
+    buf[-guard:] = 7.0
+    y = ops.gemm(a, w, sa, sb, out=buf[guard:guard + M * N].view(M, N))
+    torch.cuda.synchronize()
+    assert np.array_equal(bits16(y), ref_gemm(a, w, sa, sb))
+    assert bool((buf[:guard] == 7.0).all()) and bool((buf[-guard:] == 7.0).all())
+
+
+# one case of each form: fp16, bias, row maxima, scalar scales, strided output rows, the raw accumulator
+@pytest.mark.parametrize("form,M,N,K,tail", [c for c in CASES if c[1:3] not in ((33, 16), (320, 21504))])
+def test_form_epilogues(cuda, form, M, N, K, tail):
+    from h3_tp2_amd import ops
+    a, w, sa, sb = int_operands(M, N, K, seed=N + K, device=cuda)
+    g = torch.Generator().manual_seed(N)
+    for dt, with_bias in ((torch.bfloat16, True), (torch.float16, False), (torch.float16, True)):
+        bias = (torch.randn(N, generator=g) * 0.3).to(dt).to(cuda) if with_bias else None
+        am = torch.full((M,), -1.0, device=cuda)
+        full = torch.full((M, N + 24), 3.0, device=cuda, dtype=dt)
+        y = ops.gemm(a, w, sa[:1].reshape(()), sb, dt, bias, out=full[:, :N], row_amax=am)
+        torch.cuda.synchronize()
+        assert np.array_equal(bits16(y), ref_gemm(a, w, sa[:1].expand(M), sb, bias, dt == torch.float16))
+        assert bool((full[:, N:] == 3.0).all())
+        assert np.array_equal(f32(am), np.abs(f32(y)).max(axis=1))
+    acc = ops.gemm(a, w, sa, sb, torch.float32)
+    one = torch.ones(1, device=cuda)
+    torch.cuda.synchronize()
+    # |acc| <= 8 K, an integer: its bf16 rounding is the scaled output at unit scales
+    assert np.array_equal(bits16(acc.to(torch.bfloat16)), ref_gemm(a, w, one.expand(M), one.expand(N)))
