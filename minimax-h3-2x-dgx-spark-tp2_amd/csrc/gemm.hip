@@ -751,9 +751,15 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(GroupedParams gp) {
 // Each wave streams its weight rows at a rate bounded by its own load latency, so more, smaller waves finish sooner:
 // 16 rows per wave against 32 measured M = 2, N = 18 432, K = 3072: 11.0 -> 10.6 us; M = 5: 6.6 -> 5.8 us; M = 17:
 // 4.8 -> 4.4 us; M = 32, K = 8192: 13.9 -> 12.0 us (8 rows per wave: between the two).  A stage holds the 16 weight
-// rows and MB 8-row groups of token rows (MB = 1 for M <= 8, else 4; the lanes of token rows past 8 MB take zero
-// operands); the ring is 4 stages deep for MB = 1 and 3 for MB = 4 (12 / 18 KiB).  No other wave reads the ring, so no
-// barrier: the wave's own vmcnt wait publishes a stage and its own lgkmcnt wait releases it.
+// rows and MB 8-row groups of token rows (MB = 1 for M <= 8, else 4).  No other wave reads the ring, so no barrier: the
+// wave's own vmcnt wait publishes a stage and its own lgkmcnt wait releases it.
+// With up to 4 waves per CU the weight stream is bound by the loads in flight (from HBM) and by the k-step's own chain of
+// fragment reads, two dependent MFMAs and load issues (from the MALL): the ring is 8 stages deep (MB = 4: 6; 24 / 36
+// KiB), and a k-step reads the next one's fragments between its MFMAs and refills its slot behind them.  With more waves
+// the ring stays at 4 (MB = 4: 3) stages: deeper ones measured 5-10 % slower.  Against rings of 4 / 3 stages whose
+// fragments were read ahead of the k-step's own MFMAs, weight in the MALL / from HBM, M x N x K: 2 x 5376 x 14336
+// 19.1 / 26.4 -> 15.2 / 18.2 us, 16 x 5376 x 14336 21.9 / 30.9 -> 19.1 / 24.9, 1 x 3072 x 8192 11.3 / 13.8 -> 9.5 / 10.4,
+// 4 x 1536 x 4608 7.2 / 7.4 -> 6.2 / 6.5, 32 x 18 432 x 3072 (1152 waves) 12.8 / 18.3 -> 12.4 / 17.7.
 // Every output element goes through the same MFMA sequence as in gemm_kernel: v_mfma 32x32x64 with the weight row at
 // A-row n % 32 and the token at B-column m % 32, the 64-deep k chunks in ascending order, two per 128-deep k-step (a
 // chunk at or past K reads zeros, as the big tiles' last k-step does), and the same epilogue, so the output is bitwise
@@ -761,96 +767,118 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(GroupedParams gp) {
 constexpr int ROWS_MAX_M = 32;
 constexpr int ROWS_RW = 16;                               // weight rows per wave
 
-template <int MB>
+template <int MB, bool DEEP>
 struct RowsRing {
     static constexpr int STAGE = (ROWS_RW + 8 * MB) * ROWB;    // the weight rows, then 8 MB token rows
-    static constexpr int DEPTH = MB == 1 ? 4 : 3;
+    static constexpr int DEPTH = DEEP ? (MB == 1 ? 8 : 6) : (MB == 1 ? 4 : 3);
     static constexpr int LOADS = ROWS_RW / 8 + MB;             // LDS-DMA instructions per k-step
-    static_assert(DEPTH >= 2 && LOADS * (DEPTH - 1) <= 63, "vmcnt range");
+    static_assert(DEPTH >= 3 && LOADS * (DEPTH - 1) <= 63, "vmcnt range");
 };
 
-// NT: the weight loads carry the non-temporal hint (chosen by the launcher, see launch_rows_t).
-template <int OUT_DT, bool HAS_BIAS, bool AMAX, int MB, bool NT>
+// DEEP: at most 4 waves per CU (chosen by launch_rows_t).
+template <int OUT_DT, bool HAS_BIAS, bool AMAX, int MB, bool DEEP>
 __global__ void __launch_bounds__(64) gemm_rows_kernel(GemmParams p) {
-    constexpr int ROWS_DEPTH = RowsRing<MB>::DEPTH;
-    constexpr int ROWS_STAGE = RowsRing<MB>::STAGE;
+    constexpr bool NT = MB == 1 && !DEEP;                 // the weight loads carry the non-temporal hint (launch_rows_t)
+    constexpr int ROWS_DEPTH = RowsRing<MB, DEEP>::DEPTH;
+    constexpr int ROWS_STAGE = RowsRing<MB, DEEP>::STAGE;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[ROWS_DEPTH * ROWS_STAGE];
     const int lane = threadIdx.x;
     const int r = lane & 31, h = lane >> 5;
     const int n0 = (int)blockIdx.x * ROWS_RW;
     const uint32_t lds0 = lds_addr(lds);
-    const v4u dw = buffer_desc(p.w, p.w_bytes);
-    const v4u da = buffer_desc(p.a, p.a_bytes);
     // LDS-DMA lane layout (as make_loader): lane l moves row 8 i + (l >> 3) of an 8-row group i, LDS chunk l & 7, which
     // holds logical chunk (l & 7) ^ swz(row); swz depends on the row's bit 3, so even and odd groups differ
     const int lrow = lane >> 3;
-    const uint32_t lch[2] = {(uint32_t)((lane & 7) ^ swz(lrow)), (uint32_t)((lane & 7) ^ swz(lrow + 8))};
-    uint32_t wrow[4], arow[4];                            // byte offsets of this lane's row in each 8-row group
-                                                          // (weights: the first ROWS_RW / 8 groups)
+    uint32_t vw[ROWS_RW / 8], va[MB];                     // byte offsets at k = 0 of this lane's row in each 8-row group
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int n = n0 + 8 * i + lrow, m = 8 * i + lrow;
-        wrow[i] = n < p.N ? (uint32_t)((int64_t)n * p.ldw) : OOB;
-        arow[i] = m < p.M ? (uint32_t)((int64_t)m * p.lda) : OOB;
+    for (int i = 0; i < ROWS_RW / 8; ++i) {
+        const int n = n0 + 8 * i + lrow;
+        vw[i] = n < p.N ? (uint32_t)((int64_t)n * p.ldw) + 16u * (uint32_t)((lane & 7) ^ swz(lrow + 8 * (i & 1))) : OOB;
     }
-    const int nk = (p.K + BK - 1) / BK;
-    // the RowsRing<MB>::LOADS = ROWS_RW / 8 + MB loads of k-step ks into ring slot `slot`: pieces at or past K read
-    // zeros (K % 16 == 0)
-    auto issue = [&](int slot, int ks) {
-        const uint32_t st = lds0 + (uint32_t)slot * ROWS_STAGE;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t c = (uint32_t)ks * BK + 16u * lch[i & 1];
-            const bool in = c < (uint32_t)p.K;
-            if (i < ROWS_RW / 8) {
-                const uint32_t off = in && wrow[i] != OOB ? wrow[i] + c : OOB;
-                if (NT) dma16_nt(dw, st + (uint32_t)i * 8 * ROWB, off);
-                else dma16(dw, st + (uint32_t)i * 8 * ROWB, off);
-            }
-            if (i < MB)
-                dma16(da, st + ROWS_RW * ROWB + (uint32_t)i * 8 * ROWB, in && arow[i] != OOB ? arow[i] + c : OOB);
+    for (int i = 0; i < MB; ++i) {
+        const int m = 8 * i + lrow;
+        va[i] = m < p.M ? (uint32_t)((int64_t)m * p.lda) + 16u * (uint32_t)((lane & 7) ^ swz(lrow + 8 * (i & 1))) : OOB;
+    }
+    const int nk = (p.K + BK - 1) / BK, ktail = p.K % BK;
+    // The loads of the next k-step into ring slot `slot` (a byte offset).  The last k-step of a K that is no multiple of
+    // BK cuts the lanes past K off for good; past the last k-step the descriptors are empty (their offset too), so the
+    // loads read zeros and touch no memory.
+    v4u dw = buffer_desc(p.w, p.w_bytes), da = buffer_desc(p.a, p.a_bytes);
+    const uint32_t wbytes = dw[2], abytes = da[2];
+    int left = nk;
+    uint32_t k0 = 0;
+    auto issue = [&](uint32_t slot) {
+        if (__builtin_expect(left == 1 && ktail != 0, 0)) {
+#pragma unroll
+            for (int i = 0; i < ROWS_RW / 8; ++i)
+                if (16 * ((lane & 7) ^ swz(lrow + 8 * (i & 1))) >= ktail) vw[i] = OOB;
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+                if (16 * ((lane & 7) ^ swz(lrow + 8 * (i & 1))) >= ktail) va[i] = OOB;
         }
-    };
-    auto kstep_mfma = [&](v16f& acc, int slot) {
-        const uint8_t* st = lds + slot * ROWS_STAGE;
-        const int alane = (r % ROWS_RW) | (lane & 32);    // A rows past ROWS_RW repeat rows r % ROWS_RW
-        const v8i a0 = read_frag(st, alane, 0), a1 = read_frag(st, alane, 1);
-        v8i b0 = {0, 0, 0, 0, 0, 0, 0, 0}, b1 = b0;
-        if (MB == 4 || r < 8 * MB) {                    // token rows past 8 MB: zero operands, nothing staged
-            b0 = read_frag(st + ROWS_RW * ROWB, lane, 0);
-            b1 = read_frag(st + ROWS_RW * ROWB, lane, 1);
+        dw[2] = left > 0 ? wbytes : 0;
+        da[2] = left > 0 ? abytes : 0;
+        k0 = left > 0 ? k0 : 0;
+        const uint32_t st = lds0 + slot;
+#pragma unroll
+        for (int i = 0; i < ROWS_RW / 8; ++i) {
+            if (NT) dma16_at_nt(dw, st + (uint32_t)i * 8 * ROWB, vw[i], k0);
+            else dma16_at(dw, st + (uint32_t)i * 8 * ROWB, vw[i], k0);
         }
-        wait_lgkm0();                                   // the slot is read: the next issue may refill it
-        acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a0, b0, acc, 0, 0, 0, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a1, b1, acc, 0, 0, 0, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < MB; ++i) dma16_at(da, st + ROWS_RW * ROWB + (uint32_t)i * 8 * ROWB, va[i], k0);
+        --left;
+        k0 += BK;
     };
+    struct Frags { v8i a[2], b[2]; };
+    auto read = [&](Frags& F, uint32_t slot) {
+        // A rows past ROWS_RW repeat rows r % ROWS_RW, tokens past 8 MB repeat tokens r % (8 MB): their results are not
+        // stored, and no other's depends on them
+        const uint8_t* st = lds + slot;
+        const int alane = (r % ROWS_RW) | (lane & 32), blane = (r % (8 * MB)) | (lane & 32);
+        F.a[0] = read_frag(st, alane, 0);
+        F.b[0] = read_frag(st + ROWS_RW * ROWB, blane, 0);
+        F.a[1] = read_frag(st, alane, 1);
+        F.b[1] = read_frag(st + ROWS_RW * ROWB, blane, 1);
+    };
+    auto next = [](uint32_t slot) { return slot == (ROWS_DEPTH - 1) * ROWS_STAGE ? 0u : slot + ROWS_STAGE; };
 
     v16f acc;
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.f;
 #pragma unroll
-    for (int s = 0; s < ROWS_DEPTH; ++s) issue(s, s);
-    // every k-step issues ROWS_RW / 8 + MB loads (RowsRing::LOADS; past the last k-step out of range, touching no
-    // memory), so when k-step ks is consumed exactly the loads of the ROWS_DEPTH - 1 younger k-steps may be in flight
-    int ks = 0;
-    for (; ks + ROWS_DEPTH <= nk; ks += ROWS_DEPTH) {
-#pragma unroll
-        for (int s = 0; s < ROWS_DEPTH; ++s) {
-            __builtin_amdgcn_s_waitcnt(vmcnt_imm(RowsRing<MB>::LOADS * (ROWS_DEPTH - 1)));
-            asm volatile("" ::: "memory");
-            kstep_mfma(acc, s);
-            issue(s, ks + s + ROWS_DEPTH);
-        }
-    }
-#pragma unroll
-    for (int s = 0; s < ROWS_DEPTH - 1; ++s) {          // the last nk mod ROWS_DEPTH k-steps, already in flight
-        if (ks + s < nk) {
-            wait_vm0();
-            asm volatile("" ::: "memory");
-            kstep_mfma(acc, s);
-        }
+    for (int s = 0; s < ROWS_DEPTH; ++s) issue((uint32_t)s * ROWS_STAGE);
+    constexpr int LOADS = RowsRing<MB, DEEP>::LOADS;      // of every k-step, also past the last one
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(LOADS * (ROWS_DEPTH - 1)));
+    asm volatile("" ::: "memory");
+    Frags F, G;
+    read(F, 0);
+    uint32_t slot = 0;
+    // A k-step: the next one's fragments (all but the ROWS_DEPTH - 2 youngest have landed) are read behind its first MFMA,
+    // and its own slot, whose fragments are in registers, is refilled behind its second.
+    auto kstep = [&](const Frags& cur, Frags& nxt) {
+        wait_lgkm0();
+        acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(cur.a[0], cur.b[0], acc, 0, 0, 0, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(LOADS * (ROWS_DEPTH - 2)));
+        asm volatile("" ::: "memory");
+        const uint32_t own = slot;
+        slot = next(slot);
+        read(nxt, slot);
+        __builtin_amdgcn_sched_barrier(0);
+        acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(cur.a[1], cur.b[1], acc, 0, 0, 0, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        issue(own);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // in pairs: an odd count takes one more k-step, of zeros, which leaves the accumulators as they are
+    for (int ks = 0; ks < nk; ks += 2) {
+        kstep(F, G);
+        kstep(G, F);
     }
     wait_vm0();                                         // the out-of-range tail loads have landed before the exit
+    wait_lgkm0();
 
     // epilogue: register 4q + rr holds weight row n0 + 8q + 4h + rr for token r (the MFMA result layout); rows at or
     // past ROWS_RW are the repeated ones
@@ -892,7 +920,7 @@ __global__ void __launch_bounds__(64) gemm_rows_kernel(GemmParams p) {
     }
 }
 
-// With at least 4 waves per CU of the one-token-group form the weight stream is bandwidth-bound and its loads take the
+// With more than 4 waves per CU of the one-token-group form the weight stream is bandwidth-bound and its loads take the
 // non-temporal hint; with fewer waves (each streaming more k-steps) or the four-group form the hint made it slower.
 // Measured (one process, interleaved, median of 7, outputs identical), M x N x K: 2 x 18 432 x 3072 (1152 waves)
 // 10.6 -> 9.2 us, 2 x 36 864 x 3072 19.1 -> 17.6, 5 x 18 432 x 3072 10.5 -> 9.3; but 2 x 9216 x 3072 (576 waves)
@@ -902,14 +930,17 @@ template <int OUT_DT, bool HAS_BIAS, bool AMAX>
 int launch_rows_t(const GemmParams& p, hipStream_t st) {
     const int waves = (p.N + ROWS_RW - 1) / ROWS_RW;
     const dim3 grid((unsigned)waves);
+    const bool deep = waves <= 4 * h3host::cu_count();
+#define H3_ROWS(MB, DEEP)                                                                                   \
+    hipLaunchKernelGGL((gemm_rows_kernel<OUT_DT, HAS_BIAS, AMAX, MB, DEEP>), grid, dim3(64), 0, st, p)
     if (p.M <= 8) {
-        if (waves >= 4 * h3host::cu_count())
-            hipLaunchKernelGGL((gemm_rows_kernel<OUT_DT, HAS_BIAS, AMAX, 1, true>), grid, dim3(64), 0, st, p);
-        else
-            hipLaunchKernelGGL((gemm_rows_kernel<OUT_DT, HAS_BIAS, AMAX, 1, false>), grid, dim3(64), 0, st, p);
+        if (deep) H3_ROWS(1, true);
+        else H3_ROWS(1, false);
     } else {
-        hipLaunchKernelGGL((gemm_rows_kernel<OUT_DT, HAS_BIAS, AMAX, 4, false>), grid, dim3(64), 0, st, p);
+        if (deep) H3_ROWS(4, true);
+        else H3_ROWS(4, false);
     }
+#undef H3_ROWS
     H3_CHECK_HIP(hipGetLastError());
     return H3FP8_OK;
 }

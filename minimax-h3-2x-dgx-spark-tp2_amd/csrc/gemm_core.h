@@ -122,11 +122,11 @@ __device__ __forceinline__ void dma16_at(v4u desc, uint32_t lds_base, uint32_t v
                  : "memory", "m0");
 }
 
-// The same load with the non-temporal hint, for operands that stream through once.
-__device__ __forceinline__ void dma16_nt(v4u desc, uint32_t lds_base, uint32_t voff) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
+// ... with the non-temporal hint, for operands that stream through once.
+__device__ __forceinline__ void dma16_at_nt(v4u desc, uint32_t lds_base, uint32_t voff, uint32_t soff) {
+    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
                  :
-                 : "s"(lds_base), "v"(voff), "s"(desc)
+                 : "s"(lds_base), "v"(voff), "s"(desc), "s"(soff)
                  : "memory", "m0");
 }
 

@@ -84,3 +84,16 @@ def test_form_epilogues(cuda, form, M, N, K, tail):
     torch.cuda.synchronize()
     # |acc| <= 8 K, an integer: its bf16 rounding is the scaled output at unit scales
     assert np.array_equal(bits16(acc.to(torch.bfloat16)), ref_gemm(a, w, one.expand(M), one.expand(N)))
+
+
+# the small-M form's rings: 8 / 6 stages with at most 4 waves per CU (16 384 weight rows), 4 / 3 beyond; fewer k-steps
+# than stages, as many, one more, odd counts and a K tail
+@pytest.mark.parametrize("N", [528, 16384, 16400])
+@pytest.mark.parametrize("M,K", [(1, 16), (8, 1024), (8, 1040), (9, 768), (32, 400), (17, 896), (5, 2192)])
+def test_small_m_rings_equal_full_tiles(cuda, M, N, K):
+    from h3_tp2_amd import ops
+    a, w, sa, sb = serving_like(M, N, K, seed=M + N + K, device=cuda)
+    y = ops.gemm(a, w, sa, sb)
+    (ref,) = ops.grouped_gemm([(a, w, sa, sb)])
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
