@@ -1,4 +1,5 @@
-"""Build libh3fp8.so (the HIP kernels + C ABI) for gfx950 with hipcc, in-tree.
+"""Build libh3fp8.so (the HIP kernels + C ABI) for gfx950 with hipcc, and _host.so (the native host path of the common
+calls, a CPython extension on the installed torch) with g++, in-tree.
 
     python minimax-h3-2x-dgx-spark-tp2_amd/build.py [--jobs N] [--asm]
 
@@ -19,6 +20,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "h3_tp2_amd", "libh3fp8.so")
+HOST = os.path.join(HERE, "h3_tp2_amd", "_host.so")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 
 ARCH = "gfx950"
@@ -49,6 +51,24 @@ def _compile(src: str, asm: bool) -> str:
     return obj
 
 
+def build_host() -> str:
+    """_host.so: csrc/host.cpp against torch's headers, linked to libh3fp8.so next to it."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    root = os.environ.get("ROCM_PATH", "/opt/rocm")
+    includes = [INCLUDE, *cpp_extension.include_paths(), sysconfig.get_paths()["include"], os.path.join(root, "include")]
+    lib_dir = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = HOST + ".tmp"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+                    f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{d}" for d in includes),
+                    os.path.join(CSRC, "host.cpp"), "-o", tmp, f"-L{os.path.dirname(LIB)}", "-lh3fp8", f"-L{lib_dir}",
+                    "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", "-Wl,-rpath,$ORIGIN"], check=True)
+    os.replace(tmp, HOST)
+    return HOST
+
+
 def build(jobs: int = 4, asm: bool = False, verbose: bool = True) -> str:
     os.makedirs(BUILD, exist_ok=True)
     srcs = sources()
@@ -57,6 +77,7 @@ def build(jobs: int = 4, asm: bool = False, verbose: bool = True) -> str:
     tmp = LIB + ".tmp"
     subprocess.run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs], check=True)
     os.replace(tmp, LIB)
+    build_host()
     if verbose:
         print(f"built {LIB} from {len(srcs)} sources", file=sys.stderr)
     return LIB

@@ -11,6 +11,7 @@ import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libh3fp8.so")
+HOST_PATH = os.path.join(_HERE, "_host.so")
 ABI_VERSION = 1
 
 H3FP8_DT_BF16 = 0
@@ -104,10 +105,23 @@ def load(path: str | None = None) -> ctypes.CDLL:
         return L
 
 
+def fail(name: str, rc: int) -> None:
+    """Raise the error of a non-zero status of entry point ``name``."""
+    msg = load().h3fp8_last_error()
+    raise H3Fp8Error(name, rc, msg.decode() if msg else "")
+
+
 def call(name: str, *args) -> None:
     """Call an entry point and raise H3Fp8Error on a non-zero status."""
-    L = load()
-    rc = getattr(L, name)(*args)
+    rc = getattr(load(), name)(*args)
     if rc != 0:
-        msg = L.h3fp8_last_error()
-        raise H3Fp8Error(name, rc, msg.decode() if msg else "")
+        fail(name, rc)
+
+
+def host():  # noqa: ANN201
+    """The native host path of the common calls (csrc/host.cpp), or None where it or the library is not built: every
+    call then takes the Python path to the same kernels, and raises there if the library is missing."""
+    if not (os.path.exists(HOST_PATH) and os.path.exists(LIB_PATH)):
+        return None
+    from . import _host
+    return _host

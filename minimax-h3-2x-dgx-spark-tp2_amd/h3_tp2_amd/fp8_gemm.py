@@ -174,6 +174,11 @@ def route(a, b, scale_a, scale_b, out_dtype, bias=None, two_pass=None):  # noqa:
 def make_scaled_mm(orig):  # noqa: ANN001,ANN201
     """The replacement of ``ops.cutlass_scaled_mm``: eligible calls go to ``route``, the rest to ``orig``."""
     def _mm(a, b, scale_a, scale_b, out_dtype, bias=None):  # noqa: ANN001,ANN202
+        if _state["fused"] and not _routers and not _stash_hooks:
+            y = ops.native_scaled_mm(a, b, scale_a, scale_b, out_dtype, bias)
+            if y is not None:
+                _stats["hip"] += 1
+                return y
         if not eligible(a, b, scale_a, scale_b, out_dtype, bias):
             _stats["stock"] += 1
             return orig(a, b, scale_a, scale_b, out_dtype, bias)

@@ -22,6 +22,10 @@ MIN_SCALE = 1.0 / (FP8_MAX * 512.0)     # vLLM's minimum per-token scale (fp8_qu
 _DT = {torch.bfloat16: _lib.H3FP8_DT_BF16, torch.float16: _lib.H3FP8_DT_FP16, torch.float32: _lib.H3FP8_DT_F32}
 
 
+# The native path of the common calls: it returns None for a call that is not in the plain form it takes (or is None
+# itself where it is not built), and the code below it then checks, refuses or computes that call.
+_host = _lib.host()
+
 _RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
@@ -95,6 +99,8 @@ def init(device=None) -> None:  # noqa: ANN001
 def quant_rows(x: torch.Tensor, q: torch.Tensor | None = None, scale: torch.Tensor | None = None):
     """Dynamic per-token quant of a bf16 [M, K] tensor: (q e4m3fn [M, K], scale fp32 [M, 1]).
     Replaces ``QuantFP8.forward`` / ``fp8_quant_fuse.quant`` (h3_tp2/fp8_quant_fuse.py:318-327)."""
+    if _host is not None and q is None and scale is None and (out := _host.quant_rows(x)) is not None:
+        return out
     _need_cuda(x)
     if x.dtype != torch.bfloat16:
         raise ValueError(f"quant_rows takes bf16, got {x.dtype}")
@@ -182,6 +188,10 @@ def gemm(a: torch.Tensor, w: torch.Tensor, scale_a: torch.Tensor, scale_b: torch
     With ``row_amax`` ([M] fp32) the epilogue also reduces max |y| per row (for the next layer's quant).
     ``out_dtype=torch.float32`` returns the raw fp32 accumulator (scales ignored: the two-pass form's product, whose
     scale pass or fused consumer follows; the reference's OUT 0)."""
+    if _host is not None and out is None and row_amax is None:
+        y = _host.gemm(a, w, scale_a, scale_b, out_dtype, bias)
+        if y is not None:
+            return y
     N = w.shape[0]
     M, sa, sa_st, sb, sb_st = _gemm_args(a, w, scale_a, scale_b, N)
     if out_dtype not in _DT:
@@ -216,12 +226,20 @@ def _scale_ptr(scale: torch.Tensor) -> tuple[int, int]:
     return flat.data_ptr(), flat.stride(0)
 
 
+def native_scaled_mm(a, b, scale_a, scale_b, out_dtype, bias=None):  # noqa: ANN001,ANN201
+    """``fp8_gemm.eligible`` and the call behind it in one native step; None for a call it leaves to those two."""
+    return None if _host is None else _host.scaled_mm(a, b, scale_a, scale_b, out_dtype, bias)
+
+
 def scaled_mm_eligible(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor, scale_b: torch.Tensor,
                        out_dtype: torch.dtype, bias: torch.Tensor | None = None) -> torch.Tensor:
     """Kernel 2 on a call that passed ``fp8_gemm.eligible`` -- the dispatcher's lean host path.  That test has checked
     the dtypes (e4m3 operands, fp32 scales, bf16 / fp16 out), the shapes, ``a`` contiguous, ``b.t()`` contiguous, the
     scale and bias sizes and K, N multiples of 16; what it leaves -- every operand on ``a``'s GPU, a bias in the
     output dtype -- is checked here, and the C side checks sizes, strides and alignment again before any launch."""
+    y = native_scaled_mm(a, b, scale_a, scale_b, out_dtype, bias)
+    if y is not None:
+        return y
     dev = a.device
     if not a.is_cuda:
         raise ValueError("h3_tp2_amd kernels run on the GPU only; got a CPU tensor")
@@ -251,6 +269,8 @@ def gemm_quant(a: torch.Tensor, w: torch.Tensor, scale_a: torch.Tensor, scale_b:
                bias: torch.Tensor | None = None):
     """GEMM to bf16 y plus the per-token e4m3 quant of y fused through the epilogue's row maxima:
     returns (y bf16 [M, N], q e4m3fn [M, N], scale fp32 [M, 1])."""
+    if _host is not None and (out := _host.gemm_quant(a, w, scale_a, scale_b, bias)) is not None:
+        return out
     N = w.shape[0]
     M, sa, sa_st, sb, sb_st = _gemm_args(a, w, scale_a, scale_b, N)
     _check_bias(bias, N, a.device)
@@ -303,6 +323,10 @@ def gemm_swiglu(a: torch.Tensor, w_gate_up: torch.Tensor, scale_a: torch.Tensor,
 def gemm_swiglu_quant(a: torch.Tensor, w_gate_up: torch.Tensor, scale_a: torch.Tensor, scale_b: torch.Tensor,
                       bias: torch.Tensor | None = None, h_ws: torch.Tensor | None = None):
     """fc1 + SwiGLU + per-token requant (fp8_swiglu level 2, h3_tp2/fp8_swiglu.py:191-200): (q [M, F], scale [M, 1])."""
+    if _host is not None and h_ws is None:
+        out = _host.gemm_swiglu_quant(a, w_gate_up, scale_a, scale_b, bias)
+        if out is not None:
+            return out
     F = _gate_up_width(w_gate_up)
     M, sa, sa_st, sb, sb_st = _gemm_args(a, w_gate_up, scale_a, scale_b, 2 * F)
     _check_bias(bias, 2 * F, a.device)
@@ -374,6 +398,8 @@ def scale_swiglu_quant(x32: torch.Tensor, sa: torch.Tensor, sb: torch.Tensor, bi
 
 def silu_mul_quant(x: torch.Tensor):
     """silu_and_mul on bf16 [M, 2F] + per-token quant: (q [M, F], scale [M, 1]) (h3_tp2/fp8_quant_fuse.py:392-402)."""
+    if _host is not None and (out := _host.silu_mul_quant(x)) is not None:
+        return out
     _need_cuda(x)
     if not isinstance(x, torch.Tensor) or x.dim() != 2 or x.dtype != torch.bfloat16:
         raise ValueError("silu_mul_quant takes a bf16 [M, 2F] tensor")
@@ -419,6 +445,8 @@ def rms_quant(x: torch.Tensor, weight: torch.Tensor, shift: torch.Tensor, scale:
               indices: torch.Tensor, eps: float, ph: torch.Tensor | None = None):
     """``rms_norm_indexed_scale_shift`` + the per-token quant of its output: (fp8 [M, H], scale [M, 1]); with ``ph``
     (bf16 [M, H]) the modulated bf16 row is stored there too (h3_tp2/fp8_quant_fuse.py:330-346)."""
+    if _host is not None and ph is None and (out := _host.rms_quant(x, weight, shift, scale, indices, eps)) is not None:
+        return out
     M, H, n_index, ib = _producer_args(x, weight, (shift, scale), indices, ("shift", "scale"))
     q = torch.empty((M, H), device=x.device, dtype=E4M3)
     s = torch.empty((M, 1), device=x.device, dtype=torch.float32)
@@ -464,6 +492,10 @@ def gate_rms_quant(residual: torch.Tensor, gate: torch.Tensor, branch: torch.Ten
                    ph: torch.Tensor | None = None):
     """``indexed_gate_rms_norm_scale_shift`` with the modulated output quantised per token: (residual_out bf16 [M, H],
     fp8 [M, H], scale [M, 1]); ``ph`` as in ``rms_quant`` (h3_tp2/fp8_quant_fuse.py:349-369)."""
+    if _host is not None and ph is None:
+        out = _host.gate_rms_quant(residual, gate, branch, weight, shift, scale, indices, eps)
+        if out is not None:
+            return out
     M, H, n_index, ib = _producer_args(residual, weight, (gate, shift, scale), indices, ("gate", "shift", "scale"))
     if branch.shape != residual.shape or branch.dtype != torch.bfloat16:
         raise ValueError("branch must be bfloat16 with the residual's shape")

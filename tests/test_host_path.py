@@ -1,0 +1,131 @@
+"""The native host path of the common calls (csrc/host.cpp) against the Python path of the same functions: the same
+outputs for every form it takes, and every other form left to the Python path -- taken or refused with the same error."""
+import pytest
+import torch
+
+from _util import int_operands
+from h3_tp2_amd import _lib, fp8_gemm, ops
+
+E4M3 = torch.float8_e4m3fn
+BF16 = torch.bfloat16
+
+
+class Sub(torch.Tensor):
+    pass
+
+
+def test_leaves_cpu_tensors_subclasses_and_other_arguments_to_python():
+    h = _lib.host()
+    assert h is not None, "the native host path is not built"
+    x = torch.zeros(4, 64, dtype=BF16)
+    a, s = torch.zeros(4, 64).to(E4M3), torch.ones(4)
+    for bad in (x, None, 3, x.as_subclass(Sub)):
+        assert h.quant_rows(bad) is None and h.silu_mul_quant(bad) is None
+        assert h.gemm(bad, a, s, s, BF16, None) is None and h.scaled_mm(bad, a, s, s, BF16, None) is None
+        assert h.gemm_quant(bad, a, s, s, None) is None and h.gemm_swiglu_quant(bad, a, s, s, None) is None
+        assert h.rms_quant(bad, x, x, x, s, 1e-6) is None and h.gate_rms_quant(bad, x, x, x, x, x, s, 1e-6) is None
+    for f in (h.quant_rows, h.gemm, h.scaled_mm, h.gemm_quant, h.gemm_swiglu_quant, h.rms_quant, h.gate_rms_quant):
+        assert f() is None
+
+
+def _bits(out):
+    out = out if isinstance(out, tuple) else (out,)
+    return [(t.dtype, tuple(t.shape), t.stride(), t.contiguous().view(torch.uint8).cpu()) for t in out]
+
+
+def _result(f):
+    try:
+        return "out", _bits(f())
+    except Exception as e:  # noqa: BLE001
+        return type(e), str(e)
+
+
+def _both(monkeypatch, f):
+    """f through the native path and through the Python path alone: the same outputs, or the same refusal."""
+    got = _result(f)
+    with monkeypatch.context() as m:
+        m.setattr(ops, "_host", None)
+        ref = _result(f)
+    assert got[0] == ref[0], (got, ref)
+    if got[0] == "out":
+        assert [g[:3] for g in got[1]] == [r[:3] for r in ref[1]]
+        assert all(torch.equal(g[3], r[3]) for g, r in zip(got[1], ref[1]))
+    else:
+        assert got[1] == ref[1]
+    return got
+
+
+@pytest.mark.gpu
+def test_products_match_the_python_path(cuda, monkeypatch):
+    stock = []
+    mm = fp8_gemm.make_scaled_mm(lambda *args: stock.append(args) or args[0])
+    monkeypatch.setattr(fp8_gemm, "_state", dict(fp8_gemm._state, fused=True, level="hip"))
+    monkeypatch.setattr(fp8_gemm, "_routers", [])
+    monkeypatch.setattr(fp8_gemm, "_stash_hooks", [])
+    for M, N, K in ((1, 64, 128), (5, 96, 272), (130, 528, 1040)):
+        a, w, sa, sb = int_operands(M, N, K, seed=M, device=cuda)
+        bias = torch.randn(N, device=cuda).to(BF16)
+        wide = torch.zeros(M, K + 64, device=cuda).to(E4M3)
+        wide[:, :K] = a
+        scales = [(sa, sb), (sa.view(M, 1), sb.view(1, N)), (sa[:1], sb), (sa, sb[:1].reshape(())), (sa[:1], sb[:1]),
+                  (torch.stack((sa, sa), 1)[:, 0], torch.stack((sb, sb), 1)[:, :1]), (sa.double(), sb), (sa[:0], sb)]
+        for s_a, s_b in scales:
+            for b in (None, bias, bias.half(), bias[:-1], torch.stack((bias, bias), 1)[:, 0]):
+                for dt in (BF16, torch.float16, torch.float32):
+                    n = len(stock)
+                    _both(monkeypatch, lambda: mm(a, w.t(), s_a, s_b, dt, b))
+                    assert (len(stock) - n) % 2 == 0                  # both paths kept the stock op, or neither
+                    _both(monkeypatch, lambda: ops.gemm(a, w, s_a, s_b, dt, b))
+                _both(monkeypatch, lambda: ops.gemm_quant(a, w, s_a, s_b, b))
+                _both(monkeypatch, lambda: ops.gemm_swiglu_quant(a, w, s_a, s_b, b))
+        for x in (wide[:, :K], a[:0], a.t().contiguous().t(), a.cpu(), a.float(), a[0], a[:, :K - 8]):
+            _both(monkeypatch, lambda: ops.gemm(x, w, sa, sb))
+            _both(monkeypatch, lambda: ops.gemm_swiglu_quant(x, w, sa, sb))
+            n = len(stock)
+            if x.is_cuda:
+                _both(monkeypatch, lambda: mm(x, w.t(), sa, sb, BF16))
+                _both(monkeypatch, lambda: mm(x, w.t().contiguous(), sa, sb, BF16))
+                assert (len(stock) - n) % 2 == 0
+        assert _both(monkeypatch, lambda: ops.gemm(a, w, sa, sb))[0] == "out"
+    # a size the C side refuses: the library's error through either path
+    assert _both(monkeypatch, lambda: ops.gemm(*int_operands(4, 24, 40, 1, cuda)))[0] is _lib.H3Fp8Error
+
+
+@pytest.mark.gpu
+def test_quants_and_producers_match_the_python_path(cuda, monkeypatch):
+    g = torch.Generator(device=cuda).manual_seed(3)
+    for M, H in ((1, 64), (7, 1000), (300, 3072)):
+        wide = torch.randn(M, 2 * H, generator=g, device=cuda).to(BF16)
+        x = wide[:, :H].contiguous()
+        for t in (x, wide, wide[:, :H], wide[:, ::2], x[:0], x.float(), x[0], x.t()):
+            _both(monkeypatch, lambda: ops.quant_rows(t))
+            _both(monkeypatch, lambda: ops.silu_mul_quant(t))
+        ada = torch.randn(3, 6 * H, generator=g, device=cuda).to(BF16)
+        w = torch.randn(H, generator=g, device=cuda).to(BF16)
+        idx = torch.randint(0, 3, (M,), generator=g, device=cuda)
+        sh, sc, ga = ada[:, :H], ada[:, H:2 * H], ada[:, 2 * H:3 * H]
+        for i in (idx, idx.int(), idx.float(), torch.stack((idx, idx), 1)[:, 0], idx[:-1]):
+            for weight, eps in ((w, 1e-6), (w.view(1, H), 1e-6), (w[:-1], 1e-6), (w, 1)):
+                _both(monkeypatch, lambda: ops.rms_quant(x, weight, sh, sc, i, eps))
+                _both(monkeypatch, lambda: ops.gate_rms_quant(x, ga, wide[:, H:], weight, sh, sc, i, eps))
+        _both(monkeypatch, lambda: ops.rms_quant(x, w, sh[:, :-8], sc, idx, 1e-6))
+        _both(monkeypatch, lambda: ops.gate_rms_quant(x, ga, x[:, :-8], w, sh, sc, idx, 1e-6))
+        _both(monkeypatch, lambda: ops.gate_rms_quant(x, ga[:1], x, w, sh, sc, idx * 0, 1e-6))
+
+
+@pytest.mark.gpu
+def test_runs_on_the_current_stream_and_under_capture(cuda):
+    a, w, sa, sb = int_operands(40, 96, 256, seed=1, device=cuda)
+    ref = ops.gemm(a, w, sa, sb)
+    x = torch.randn(40, 256, device=cuda).to(BF16)
+    q_ref, s_ref = ops.quant_rows(x)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = ops.gemm(a, w, sa, sb)
+        q, s = ops.quant_rows(x)
+    for _ in range(3):
+        y.zero_()
+        s.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, ref) and torch.equal(s, s_ref) and torch.equal(q.view(torch.uint8), q_ref.view(torch.uint8))
