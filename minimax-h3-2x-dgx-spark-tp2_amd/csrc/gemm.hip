@@ -64,8 +64,6 @@ constexpr int A_REGION = BN * ROWB;             // activation rows start after t
 // The stages are never used by the epilogue, so the loads of the next tile run under it.
 constexpr int SCALE_SET = 2 * 256 * 4;
 constexpr int NSCALE = 3;
-constexpr int SILU_LDS_BYTES = H3_SILU_ROT_LEN * 2;          // the compact SiLU table (kernel 3)
-static_assert(SILU_LDS_BYTES % 256 == 0, "the table loads in 256-byte pieces");
 
 // The layout per epilogue: kernel 3 stages 16 token rows per flush (2 KiB per wave) to make room for the compact SiLU
 // table, which brings its workgroup to the 160 KiB of the CU; the other forms stage 32 rows.
@@ -360,14 +358,6 @@ __device__ __forceinline__ void kstep(uint8_t* lds, uint32_t lds0, int g, const 
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-}
-
-// A +0 the compiler cannot see through, made once per epilogue: x + z turns -0 into +0 (round to nearest) and leaves
-// every other value (NaN included) unchanged, and the add is not folded away.
-__device__ __forceinline__ float opaque_zero() {
-    float z = 0.0f;
-    asm volatile("" : "+v"(z));
-    return z;
 }
 
 // ---- epilogue ----
@@ -995,17 +985,13 @@ int dispatch(const GroupedParams& gp, int out_dt, bool has_bias, hipStream_t st)
 //   * else full tiles in whole rounds, the last partial round cut into smaller tiles if at most half the CUs have one
 //     (T mod G <= G / 2); a fuller last round runs as full tiles.  Against a tail of four-wave 256 x 128 tiles:
 //     4100 x 5376 x 14336 255.0 -> 242.6 us (101 tiles left), 16 740 x 9216 x 3072 372.7 -> 364.1 (72 left).
-// Kernel 3 (SwiGLU pairs gate and up rows inside a tile) always runs full tiles.
 int launch_split(GroupedParams gp, int epi, int out_dt, bool has_bias, hipStream_t st) {
     const GemmParams& p = gp.g[0];
     const int T = p.tiles_m * p.tiles_n;
     const int G = h3host::cu_count();
-    if (epi == EPI_SWIGLU) {
-        gp.total_tiles = T;
-        return dispatch<EPI_SWIGLU>(gp, H3FP8_DT_BF16, has_bias, st);
-    }
-    const int form = tile_form_for(p.M, p.N, G);
-    if (form < TILE_FORMS) return launch_tiles(p, form, out_dt, st);
+    const bool swiglu = epi == EPI_SWIGLU;
+    const int form = tile_form_for(p.M, p.w_rows, swiglu, G);
+    if (form < TILE_FORMS) return launch_tiles(p, form, out_dt, swiglu, st);
     const int full = (T / G) * G;
     const int rest = T - full;
     // the tail's tile map takes the full-tile launch to have covered the first full / 8 positions of each per-XCD range,
@@ -1013,10 +999,11 @@ int launch_split(GroupedParams gp, int epi, int out_dt, bool has_bias, hipStream
     // keeps full tiles throughout
     const bool tail = rest > 0 && 2 * rest <= G && full % 8 == 0;
     gp.total_tiles = tail ? full : T;
-    const int rc = epi == EPI_PLAIN ? dispatch<EPI_PLAIN>(gp, out_dt, has_bias, st)
-                                    : dispatch<EPI_AMAX>(gp, out_dt, has_bias, st);
+    const int rc = swiglu             ? dispatch<EPI_SWIGLU>(gp, H3FP8_DT_BF16, has_bias, st)
+                   : epi == EPI_PLAIN ? dispatch<EPI_PLAIN>(gp, out_dt, has_bias, st)
+                                      : dispatch<EPI_AMAX>(gp, out_dt, has_bias, st);
     if (rc || !tail) return rc;
-    return launch_tile_tail(p, full, rest, G, out_dt, st);
+    return launch_tile_tail(p, full, rest, G, out_dt, swiglu, st);
 }
 
 constexpr int64_t kMaxBufferBytes = 0x7fff0000LL;   // buffer offsets are 32-bit; keep clear of the OOB marker

@@ -180,15 +180,27 @@ __device__ __forceinline__ uint32_t pk_max_f32(u16x2 m) {
     return (a > b ? a : b) << 16;
 }
 
+// A +0 the compiler cannot see through, made once per epilogue: x + z turns -0 into +0 (round to nearest) and leaves
+// every other value (NaN included) unchanged, and the add is not folded away.
+__device__ __forceinline__ float opaque_zero() {
+    float z = 0.0f;
+    asm volatile("" : "+v"(z));
+    return z;
+}
+
+constexpr int SILU_LDS_BYTES = H3_SILU_ROT_LEN * 2;          // the compact SiLU table (kernel 3)
+static_assert(SILU_LDS_BYTES % 256 == 0, "the table loads in 256-byte pieces");
+
 // gemm_tile.hip: the forms of smaller tiles, one per workgroup, in ascending order of their area.
 enum TileForm { TILE_32x64, TILE_64x64, TILE_96x64, TILE_128x64, TILE_128x128, TILE_192x128, TILE_256x128, TILE_FORMS };
 
-// The first form whose tiles over an M x N output number at most `limit` (TILE_FORMS: none).
-int tile_form_for(int64_t M, int64_t N, int64_t limit);
+// The first form whose tiles over M tokens x w_rows weight rows number at most `limit` (TILE_FORMS: none).  swiglu: the
+// tiles of kernel 3 (w_rows = 2F), which has some of the forms only.
+int tile_form_for(int64_t M, int64_t w_rows, bool swiglu, int64_t limit);
 // The whole problem in tiles of one form.
-int launch_tiles(GemmParams p, int form, int out_dt, hipStream_t st);
+int launch_tiles(GemmParams p, int form, int out_dt, bool swiglu, hipStream_t st);
 // What a launch over the first `first` 256 x 256 tiles of the problem has left (`rest` of them), each cut into the same
 // number of tiles of the smallest form that keeps all of them within `limit` workgroups.
-int launch_tile_tail(GemmParams p, int first, int rest, int limit, int out_dt, hipStream_t st);
+int launch_tile_tail(GemmParams p, int first, int rest, int limit, int out_dt, bool swiglu, hipStream_t st);
 
 }  // namespace h3g

@@ -21,13 +21,18 @@ namespace {
 using namespace h3g;
 
 // NST: k-steps of the ring.  KS: k-steps per barrier.
-template <int WN_, int WM_, int NI_, int NJ_, int NST_, int KS_>
+// SW: the tile of kernel 3, whose TW weight rows are TW / 2 gate rows and the matching up rows; a wave's first NI / 2
+// blocks are gate rows, the others the up rows of the same channels.
+template <int WN_, int WM_, int NI_, int NJ_, int NST_, int KS_, bool SW_ = false>
 struct Tile {
     static constexpr int WN = WN_, WM = WM_, NI = NI_, NJ = NJ_, NST = NST_, KS = KS_;
+    static constexpr bool SW = SW_;
+    static_assert(!SW || NI % 2 == 0, "gate and up blocks in pairs");
     static_assert(NST >= 2 * KS, "ring depth");
     static constexpr int WAVES = WN * WM;
     static constexpr int TW = 32 * NI * WN;              // weight rows per tile
     static constexpr int TT = 32 * NJ * WM;              // token rows per tile
+    static constexpr int TC = SW ? TW / 2 : TW;          // output channels per tile
     static constexpr int WG = TW / 8, AG = TT / 8;       // 8-row load groups of a stage
     static constexpr int WL = (WG + WAVES - 1) / WAVES, AL = (AG + WAVES - 1) / WAVES;   // per wave
     static constexpr int LOADS = WL + AL;
@@ -37,8 +42,13 @@ struct Tile {
     static constexpr int SCALES_OFF = NST * STAGE;
     static constexpr int JUNK_OFF = SCALES_OFF + (SA_N + SB_N) * 4;
     static constexpr bool JUNK = WG % WAVES != 0 || AG % WAVES != 0;
-    static constexpr int LDS = JUNK_OFF + (JUNK ? 1024 : 0);
-    static constexpr int STG_PER_WAVE = 32 * (NI * 128 + 16);   // the fp32 output's; 16-bit outputs use half
+    static constexpr int STG_PER_WAVE = 32 * ((SW ? NI * 32 : NI * 128) + 16);   // SW: NI / 2 blocks of bf16; else of fp32
+    // SW: the compact SiLU table, next to the ring where it fits, else behind the staging area once the ring is free
+    static constexpr int END = (JUNK_OFF + (JUNK ? 1024 : 0) + 255) / 256 * 256;
+    static constexpr bool SILU_LATE = SW && END + SILU_LDS_BYTES > 160 * 1024;
+    static constexpr int SILU_OFF = SILU_LATE ? (STG_PER_WAVE * WAVES + 255) / 256 * 256 : END;
+    static constexpr int LDS = SW && !SILU_LATE ? END + SILU_LDS_BYTES : END;
+    static_assert(!SILU_LATE || SILU_OFF + SILU_LDS_BYTES <= NST * STAGE, "the table in the ring");
     static_assert(LDS <= 160 * 1024, "LDS of one CU");
     static_assert(STG_PER_WAVE * WAVES <= NST * STAGE, "the epilogue stages in the ring");
     static_assert(LOADS * (NST - 1) <= 63, "vmcnt range");
@@ -57,6 +67,14 @@ struct TileLoader {
     int ktail;                                           // K % BK
 };
 
+// The global weight row of row r of tile column tn, -1 past the last.
+template <class T>
+__device__ __forceinline__ int64_t tile_weight_row(const GemmParams& p, int tn, int r) {
+    const int up = T::SW && r >= T::TW / 2;
+    const int64_t n = T::SW ? (int64_t)tn * (T::TW / 2) + r - up * (T::TW / 2) : (int64_t)tn * T::TW + r;
+    return n < p.N ? n + (up ? p.N : 0) : -1;
+}
+
 template <class T>
 __device__ __forceinline__ void tile_loader_set(TileLoader<T>& L, const GemmParams& p, int tm, int tn, int wave,
                                                 int lane) {
@@ -73,8 +91,8 @@ __device__ __forceinline__ void tile_loader_set(TileLoader<T>& L, const GemmPara
 #pragma unroll
     for (int j = 0; j < T::WL; ++j) {
         const int g = wave * T::WL + j;
-        const int64_t row = (int64_t)tn * T::TW + 8 * g + lrow;
-        const bool ok = g < T::WG && row < p.N;
+        const int64_t row = tile_weight_row<T>(p, tn, 8 * g + lrow);
+        const bool ok = g < T::WG && row >= 0;
         L.vw[j] = ok ? (uint32_t)(row * p.ldw) + 16u * (uint32_t)((lane & 7) ^ swz(8 * (g & 1) + lrow)) : OOB;
     }
 #pragma unroll
@@ -129,11 +147,18 @@ struct Frags {
     v8i a[2][T::NI], b[2][T::NJ];
 };
 
+// The tile row of weight block i of wave column wn.
+template <class T>
+__device__ __forceinline__ int tile_block_row(int wn, int i) {
+    if (!T::SW) return (wn * T::NI + i) * 32;
+    return i < T::NI / 2 ? (wn * T::NI / 2 + i) * 32 : T::TW / 2 + (wn * T::NI / 2 + i - T::NI / 2) * 32;
+}
+
 template <class T>
 __device__ __forceinline__ void tile_read(Frags<T>& F, const uint8_t* stage, int wn, int wm, int lane, int f) {
     const int sub = f / (T::NI + T::NJ), r = f % (T::NI + T::NJ);
     if (r < T::NJ) F.b[sub][r] = read_frag(stage + T::A_OFF + (wm * T::NJ + r) * 32 * ROWB, lane, sub);
-    else F.a[sub][r - T::NJ] = read_frag(stage + (wn * T::NI + r - T::NJ) * 32 * ROWB, lane, sub);
+    else F.a[sub][r - T::NJ] = read_frag(stage + tile_block_row<T>(wn, r - T::NJ) * ROWB, lane, sub);
 }
 
 template <class T>
@@ -174,23 +199,53 @@ __device__ __forceinline__ void tile_kstep(const uint8_t* lds, uint32_t lds0, ui
     if (LOAD) tile_loader_next(L);
 }
 
+// The 32 staged token rows from m0 on (CH 16-byte chunks each, at a stride padded by 16 bytes) to their output rows, chunk
+// c of row t by lane (CH t + c) % 64 of instruction (CH t + c) / 64, so that every store writes whole row segments (the
+// store path handles about one 128-byte line per cycle: the lines an instruction touches are what it costs).  Rows past M
+// fall outside the output descriptor's range, columns past N get an out-of-range offset.
+template <int CH, int ELEM, bool MAY_NT>
+__device__ __forceinline__ void tile_store(const GemmParams& p, __amdgpu_buffer_rsrc_t yr, int col0, int m0, int lane,
+                                           const uint8_t* stg) {
+    constexpr int NS = 32 * CH / 64;
+    static_assert((32 * CH) % 64 == 0, "whole store instructions per block row");
+    const uint32_t row = (uint32_t)p.ldy * ELEM;
+    wave_sync();                                         // every lane's writes before any lane's reads
+    v4u v[NS];
+    uint32_t off[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {                       // all reads before the first store
+        const int idx = 64 * s + lane, t = idx / CH, c = idx - t * CH;
+        v[s] = *reinterpret_cast<const v4u*>(stg + t * (CH * 16 + 16) + c * 16);
+        const int n = col0 + c * (16 / ELEM);
+        off[s] = (n < p.N) ? (uint32_t)(m0 + t) * row + (uint32_t)n * ELEM : OOB;
+    }
+    if (MAY_NT && p.y_nt) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) __builtin_amdgcn_raw_buffer_store_b128(v[s], yr, off[s], 0, 2);
+    } else {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) __builtin_amdgcn_raw_buffer_store_b128(v[s], yr, off[s], 0, 0);
+    }
+}
+
+// The row maximum of token m from the two lanes that hold its channels.
+__device__ __forceinline__ void tile_row_amax(const GemmParams& p, int m, uint32_t v, int lane) {
+    const uint32_t o = (uint32_t)__shfl_xor((int)v, 32, 64);
+    v = v > o ? v : o;
+    if (lane < 32 && m < p.M && v) atomicMax(reinterpret_cast<unsigned int*>(p.row_amax) + m, v);
+}
+
 // Block (i, j) of a wave's accumulators: register 4q + r is channel col0 + 32 i + 8 q + 4 (lane >> 5) + r of token
 // mrow0 + 32 j + (lane & 31); sa_l and sb_l (LDS) hold the scales of the wave's tokens and channels.  The 32 tokens of a
-// block row j go through the wave's LDS area `stg` (rows of NI x 32 outputs at a stride padded by 16 bytes) and come back
-// as 16-byte chunks, chunk c of row t at lane (CH t + c) % 64 of instruction (CH t + c) / 64, so that every store writes
-// whole row segments (the store path handles about one 128-byte line per cycle: the lines an instruction touches are what
-// it costs).  Rows past M fall outside the output descriptor's range, columns past N get an out-of-range offset.
+// block row j go through the wave's LDS area `stg`, rows of NI x 32 outputs.
 template <int OUT_DT, int NI, int NJ>
 __device__ __forceinline__ void tile_epilogue(const GemmParams& p, int col0, int mrow0, const float* sa_l,
                                               const float* sb_l, int lane, const v16f (&acc)[NI][NJ], uint8_t* stg) {
     constexpr int ELEM = OUT_DT == H3FP8_DT_F32 ? 4 : 2;
     constexpr int CH = NI * 2 * ELEM;                    // 16-byte chunks per staged token row
     constexpr int RS = CH * 16 + 16;                     // staged row stride (padded: rows fall on other banks)
-    constexpr int NS = 32 * CH / 64;                     // store instructions per block row
-    static_assert((32 * CH) % 64 == 0, "whole store instructions per block row");
     const int hi = lane >> 5, mj = lane & 31;
     const __amdgpu_buffer_rsrc_t yr = make_rsrc(p.y, p.y_bytes);
-    const uint32_t row = (uint32_t)p.ldy * ELEM;
     const bool has_bias = p.bias != nullptr, amax = p.row_amax != nullptr;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
@@ -234,28 +289,83 @@ __device__ __forceinline__ void tile_epilogue(const GemmParams& p, int col0, int
                 const v2u32 val = {lo, hi2};
                 *reinterpret_cast<v2u32*>(stg + mj * RS + (4 * i + q) * 16 + 8 * hi) = val;
             }
-        wave_sync();                                     // every lane's writes before any lane's reads
-        v4u v[NS];
-        uint32_t off[NS];
+        tile_store<CH, ELEM, OUT_DT == H3FP8_DT_F32>(p, yr, col0, mrow0 + 32 * j, lane, stg);
+        if (amax) tile_row_amax(p, m, rmax, lane);
+    }
+}
+
+// Kernel 3's: blocks (t, j) and (NT + t, j) are the gate and the up of channels col0 + 32 t + ...; sb_l holds the gate
+// scales and, up_off entries on, the up scales.  The arithmetic and the SiLU lookup (the compact table `silu_l`, or the
+// full one for a block with a gate outside its range) are those of the 256 x 256 tiles.
+template <int NT, int NJ>
+__device__ __forceinline__ void swiglu_epilogue(const GemmParams& p, int col0, int mrow0, const float* sa_l,
+                                                const float* sb_l, int up_off, const uint16_t* silu_l, int lane,
+                                                const v16f (&acc)[2 * NT][NJ], uint8_t* stg) {
+    constexpr int CH = NT * 4, RS = CH * 16 + 16;
+    const int hi = lane >> 5, mj = lane & 31;
+    const __amdgpu_buffer_rsrc_t yr = make_rsrc(p.y, p.y_bytes);
+    const bool has_bias = p.bias != nullptr, amax = p.row_amax != nullptr;
+    const float zero = opaque_zero();
 #pragma unroll
-        for (int s = 0; s < NS; ++s) {                   // all reads before the first store
-            const int idx = 64 * s + lane, t = idx / CH, c = idx - t * CH;
-            v[s] = *reinterpret_cast<const v4u*>(stg + t * RS + c * 16);
-            const int n = col0 + c * (16 / ELEM);
-            off[s] = (n < p.N) ? (uint32_t)(mrow0 + 32 * j + t) * row + (uint32_t)n * ELEM : OOB;
-        }
-        if (OUT_DT == H3FP8_DT_F32 && p.y_nt) {
+    for (int j = 0; j < NJ; ++j) {
+        const int m = mrow0 + 32 * j + mj;
+        const float sam = sa_l[32 * j + mj];
+        uint32_t rmax = 0;
+        wave_sync();                                     // the previous block row's reads before these writes
 #pragma unroll
-            for (int s = 0; s < NS; ++s) __builtin_amdgcn_raw_buffer_store_b128(v[s], yr, off[s], 0, 2);
-        } else {
+        for (int t = 0; t < NT; ++t) {
+            uint32_t key[4][4], uu[4][4], sl[4][4];
+            uint64_t outside = 0;
 #pragma unroll
-            for (int s = 0; s < NS; ++s) __builtin_amdgcn_raw_buffer_store_b128(v[s], yr, off[s], 0, 0);
+            for (int q = 0; q < 4; ++q) {
+                const int c = 32 * t + 8 * q + 4 * hi, f = col0 + c;
+                const v4f sbg = *reinterpret_cast<const v4f*>(sb_l + c);
+                const v4f sbu = *reinterpret_cast<const v4f*>(sb_l + up_off + c);
+                const int fc = f < p.N ? f : 0;          // columns past F read column 0 of the bias (not stored)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float tg = sbg[r] * acc[t][j][4 * q + r], tu = sbu[r] * acc[NT + t][j][4 * q + r];
+                    float gy, uy;
+                    if (has_bias) {                      // uniform
+                        gy = __builtin_fmaf(sam, tg, load_bias(p.bias, fc + r, 0));
+                        uy = __builtin_fmaf(sam, tu, load_bias(p.bias, p.N + fc + r, 0));
+                    } else {
+                        gy = sam * tg;
+                        uy = sam * tu;
+                    }
+                    uu[q][r] = cvt_bf16x2(0.0f, uy);
+                    key[q][r] = ((cvt_bf16x2(gy, gy) >> 15) & 0xffffu) - H3_SILU_ROT_R0;
+                    outside |= __ballot(key[q][r] >= (uint32_t)H3_SILU_ROT_LEN);
+                }
+            }
+            if (outside == 0) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sl[q][r] = silu_l[key[q][r]];
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const uint32_t rk = (key[q][r] + H3_SILU_ROT_R0) & 0xffffu;
+                        sl[q][r] = p.silu[(rk >> 1) | ((rk & 1u) << 15)];
+                    }
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float hv[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r)              // -0 up -> +0 (fp8_swiglu.py:66)
+                    hv[r] = bf16_to_f32(sl[q][r]) * (u2f(uu[q][r]) + zero);
+                const v2u32 val = {cvt_bf16x2(hv[0], hv[1]), cvt_bf16x2(hv[2], hv[3])};
+                if (amax && col0 + 32 * t + 8 * q + 4 * hi < p.N)
+                    rmax = max_abs_bf16x2(max_abs_bf16x2(rmax, val[0]), val[1]);
+                *reinterpret_cast<v2u32*>(stg + mj * RS + (4 * t + q) * 16 + 8 * hi) = val;
+            }
         }
-        if (amax) {
-            const uint32_t o = (uint32_t)__shfl_xor((int)rmax, 32, 64);
-            rmax = rmax > o ? rmax : o;
-            if (hi == 0 && m < p.M && rmax) atomicMax(reinterpret_cast<unsigned int*>(p.row_amax) + m, rmax);
-        }
+        tile_store<CH, 2, false>(p, yr, col0, mrow0 + 32 * j, lane, stg);
+        if (amax) tile_row_amax(p, m, rmax, lane);
     }
 }
 
@@ -298,7 +408,7 @@ __global__ void __launch_bounds__(T::WAVES * 64, 2) gemm_tile_kernel(GemmParams 
     int tm, tn;
     if (p.tail_first >= 0) {                             // uniform
         tail_tile_of<256 / T::TW, 256 / T::TT>(p, (int)blockIdx.x, (int)gridDim.x, tm, tn);
-        if (tm * T::TT >= p.M || tn * T::TW >= p.N) return;      // a piece past the edge of its 256 x 256 tile's rows
+        if (tm * T::TT >= p.M || tn * T::TC >= p.N) return;      // a piece past the edge of its 256 x 256 tile's rows
     } else {
         const int tiles_m = (p.M + T::TT - 1) / T::TT;
         tile_of((int)blockIdx.x, (int)gridDim.x, tiles_m, (int)gridDim.x / tiles_m, TILE_GROUP_M, tm, tn);
@@ -314,11 +424,18 @@ __global__ void __launch_bounds__(T::WAVES * 64, 2) gemm_tile_kernel(GemmParams 
                 const int64_t r = (int64_t)tm * T::TT + 64 * c + lane;
                 dma4(rsa, dst, r < p.M ? (uint32_t)(r * p.sa_stride * 4) : OOB);
             } else {
-                const int64_t r = (int64_t)tn * T::TW + 64 * c - T::SA_N + lane;
-                dma4(rsb, dst, r < p.N ? (uint32_t)(r * p.sb_stride * 4) : OOB);
+                const int e = 64 * c - T::SA_N + lane;
+                const int64_t r = e < T::TW ? tile_weight_row<T>(p, tn, e) : -1;
+                dma4(rsb, dst, r >= 0 ? (uint32_t)(r * p.sb_stride * 4) : OOB);
             }
         }
     }
+    auto load_silu = [&]() {                              // 256 bytes per load, dealt over the waves
+        const v4u td = buffer_desc(p.silu_rot, SILU_LDS_BYTES);
+        for (int c = wave; c < SILU_LDS_BYTES / 256; c += T::WAVES)
+            dma4(td, lds0 + T::SILU_OFF + (uint32_t)c * 256u, (uint32_t)c * 256u + 4u * (uint32_t)lane);
+    };
+    if (T::SW && !T::SILU_LATE) load_silu();
 #pragma unroll
     for (int s = 0; s < T::NST; ++s) {
         tile_loader_edge(L, wave, lane);
@@ -373,6 +490,18 @@ __global__ void __launch_bounds__(T::WAVES * 64, 2) gemm_tile_kernel(GemmParams 
     wait_vm0();
     barrier_nofence();
     const float* sa_l = reinterpret_cast<const float*>(lds + T::SCALES_OFF);
+    if constexpr (T::SW) {
+        if (T::SILU_LATE) {
+            load_silu();
+            wait_vm0();
+            barrier_nofence();
+        }
+        swiglu_epilogue<T::NI / 2, T::NJ>(p, tn * T::TC + wn * T::NI * 16, tm * T::TT + wm * T::NJ * 32,
+                                          sa_l + wm * T::NJ * 32, sa_l + T::SA_N + wn * T::NI * 16, T::TC,
+                                          reinterpret_cast<const uint16_t*>(lds + T::SILU_OFF), lane, acc,
+                                          lds + wave * T::STG_PER_WAVE);
+        return;
+    }
     tile_epilogue<OUT_DT, T::NI, T::NJ>(p, tn * T::TW + wn * T::NI * 32, tm * T::TT + wm * T::NJ * 32,
                                         sa_l + wm * T::NJ * 32, sa_l + T::SA_N + wn * T::NI * 32, lane, acc,
                                         lds + wave * T::STG_PER_WAVE);
@@ -392,6 +521,16 @@ __global__ void __launch_bounds__(T::WAVES * 64, 2) gemm_tile_kernel(GemmParams 
     X(TILE_192x128, 2, 4, 3, 1, 3, 1)                                                                                  \
     X(TILE_256x128, 4, 2, 2, 2, 3, 1)
 
+// Kernel 3's forms: the ring of 256 x 128 leaves the compact SiLU table no room, so that form loads it at its end.
+#define H3_SWIGLU_FORMS(X)                                                                                             \
+    X(TILE_64x64, 1, 2, 2, 1, 7, 2, true)                                                                              \
+    X(TILE_128x64, 2, 2, 2, 1, 5, 2, true)                                                                             \
+    X(TILE_128x128, 2, 4, 2, 1, 4, 1, true)                                                                            \
+    X(TILE_192x128, 3, 4, 2, 1, 3, 1, true)                                                                            \
+    X(TILE_256x128, 4, 2, 2, 2, 3, 1, true)
+
+constexpr bool swiglu_form(int form) { return form != TILE_32x64 && form != TILE_96x64; }
+
 struct FormDims { int tw, tt; };
 constexpr FormDims kForms[TILE_FORMS] = {
 #define X(id, WN, WM, NI, NJ, NST, KS) {32 * WN * NI, 32 * WM * NJ},
@@ -409,11 +548,24 @@ int launch_form(const GemmParams& p, int64_t tiles, int out_dt, hipStream_t st) 
     return H3FP8_OK;
 }
 
-int launch_any(const GemmParams& p, int form, int64_t tiles, int out_dt, hipStream_t st) {
-    switch (form) {
-#define X(id, ...) case id: return launch_form<Tile<__VA_ARGS__>>(p, tiles, out_dt, st);
-        H3_TILE_FORMS(X)
+int launch_any(const GemmParams& p, int form, int64_t tiles, int out_dt, bool swiglu, hipStream_t st) {
+    if (swiglu) {
+        switch (form) {
+#define X(id, ...)                                                                                                     \
+    case id:                                                                                                           \
+        hipLaunchKernelGGL((gemm_tile_kernel<H3FP8_DT_BF16, Tile<__VA_ARGS__>>), dim3((unsigned)tiles),                \
+                           dim3(Tile<__VA_ARGS__>::WAVES * 64), 0, st, p);                                             \
+        H3_CHECK_HIP(hipGetLastError());                                                                               \
+        return H3FP8_OK;
+            H3_SWIGLU_FORMS(X)
 #undef X
+        }
+    } else {
+        switch (form) {
+#define X(id, ...) case id: return launch_form<Tile<__VA_ARGS__>>(p, tiles, out_dt, st);
+            H3_TILE_FORMS(X)
+#undef X
+        }
     }
     h3host::set_error("bad tile form %d", form);
     return H3FP8_EINVAL;
@@ -429,25 +581,25 @@ int64_t tile_count(int form, int64_t M, int64_t N) {
 
 namespace h3g {
 
-int tile_form_for(int64_t M, int64_t N, int64_t limit) {
+int tile_form_for(int64_t M, int64_t w_rows, bool swiglu, int64_t limit) {
     int f = 0;
-    while (f < TILE_FORMS && tile_count(f, M, N) > limit) ++f;
+    while (f < TILE_FORMS && ((swiglu && !swiglu_form(f)) || tile_count(f, M, w_rows) > limit)) ++f;
     return f;
 }
 
-int launch_tiles(GemmParams p, int form, int out_dt, hipStream_t st) {
+int launch_tiles(GemmParams p, int form, int out_dt, bool swiglu, hipStream_t st) {
     p.tail_first = -1;
-    return launch_any(p, form, tile_count(form, p.M, p.N), out_dt, st);
+    return launch_any(p, form, tile_count(form, p.M, p.w_rows), out_dt, swiglu, st);
 }
 
-int launch_tile_tail(GemmParams p, int first, int rest, int limit, int out_dt, hipStream_t st) {
+int launch_tile_tail(GemmParams p, int first, int rest, int limit, int out_dt, bool swiglu, hipStream_t st) {
     p.tail_first = first;
     int f = 0, pieces = 0;
     for (; f < TILE_FORMS; ++f) {
         pieces = 256 / kForms[f].tw * (256 / kForms[f].tt);
-        if (256 % kForms[f].tw == 0 && (int64_t)rest * pieces <= limit) break;
+        if (256 % kForms[f].tw == 0 && !(swiglu && !swiglu_form(f)) && (int64_t)rest * pieces <= limit) break;
     }
-    return launch_any(p, f, (int64_t)rest * pieces, out_dt, st);
+    return launch_any(p, f, (int64_t)rest * pieces, out_dt, swiglu, st);
 }
 
 }  // namespace h3g

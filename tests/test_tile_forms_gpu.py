@@ -11,6 +11,7 @@ import pytest
 import torch
 
 from _util import bits16, f32, int_operands, ref_gemm, serving_like
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -27,12 +28,12 @@ def _count(form, M, N):
     return -(-M // tt) * -(-N // tw)
 
 
-def _takes(form, M, N, tail):
+def _takes(form, M, N, tail, forms=range(len(FORMS))):
     G = torch.cuda.get_device_properties(0).multi_processor_count
     if not tail:
-        return min((f for f in range(len(FORMS)) if _count(f, M, N) <= G), default=None) == form
+        return min((f for f in forms if _count(f, M, N) <= G), default=None) == form
     rest = -(-M // 256) * -(-N // 256) % G
-    pieces = [(f, 256 // tw * (256 // tt)) for f, (tw, tt) in enumerate(FORMS) if 256 % tw == 0]
+    pieces = [(f, 256 // FORMS[f][0] * (256 // FORMS[f][1])) for f in forms if 256 % FORMS[f][0] == 0]
     return 0 < 2 * rest <= G and min(f for f, p in pieces if rest * p <= G) == form
 
 
@@ -84,6 +85,40 @@ def test_form_epilogues(cuda, form, M, N, K, tail):
     torch.cuda.synchronize()
     # |acc| <= 8 K, an integer: its bf16 rounding is the scaled output at unit scales
     assert np.array_equal(bits16(acc.to(torch.bfloat16)), ref_gemm(a, w, one.expand(M), one.expand(N)))
+
+
+# kernel 3's forms: the same tiles with gate and up rows in pairs (N = 2F)
+SWIGLU_FORMS = (1, 3, 4, 5, 6)
+SWIGLU = [(1, 1, 64, 16, False), (1, 40, 1008, 272, False), (3, 300, 2000, 400, False), (4, 600, 2000, 144, False),
+          (5, 1000, 2320, 640, False), (6, 1250, 2992, 192, False),
+          (1, 2000, 4208, 128, True), (3, 5600, 1648, 272, True), (4, 20200, 496, 96, True), (6, 22600, 496, 400, True)]
+
+
+@pytest.mark.parametrize("form,M,F,K,tail", SWIGLU)
+@pytest.mark.parametrize("bias", [False, True])
+def test_swiglu_form_equals_oracle_of_the_accumulator(cuda, form, M, F, K, tail, bias):
+    """h and the row maxima against the oracle's SwiGLU of the kernel's own fp32 accumulator, bit for bit; some rows'
+    gates are zero or far outside the compact SiLU table (those blocks take the full table), the output has guards."""
+    from h3_tp2_amd import ops
+    assert _takes(form, M, 2 * F, tail, SWIGLU_FORMS)
+    a, w, sa, sb = serving_like(M, 2 * F, K, seed=M + F, device=cuda)
+    sa = sa.clone()
+    sa[5::37] = 0.0
+    sa[11::41] *= 1e7
+    b = (torch.randn(2 * F, generator=torch.Generator().manual_seed(F)) * 0.5).to(torch.bfloat16).to(cuda) if bias else None
+    acc = ops.gemm(a, w, sa, sb, torch.float32)
+    guard = 4096
+    buf = torch.full((M * F + 2 * guard,), 7.0, device=cuda, dtype=torch.bfloat16)
+    am = torch.full((M,), -1.0, device=cuda)
+    h = ops.gemm_swiglu(a, w, sa, sb, b, row_amax=am, out=buf[guard:guard + M * F].view(M, F))
+    torch.cuda.synchronize()
+    ref = O.scale_swiglu(f32(acc), f32(sa), f32(sb), bits16(b) if bias else None)
+    got = bits16(h)
+    nan = (ref & 0x7FFF) > 0x7F80
+    assert np.array_equal((got & 0x7FFF) > 0x7F80, nan) and np.array_equal(got[~nan], ref[~nan])
+    assert bool((buf[:guard] == 7.0).all()) and bool((buf[-guard:] == 7.0).all())
+    if not nan.any():
+        assert torch.equal(am, h.float().abs().amax(dim=1))
 
 
 # the small-M form's rings: 8 / 6 stages with at most 4 waves per CU (16 384 weight rows), 4 / 3 beyond; fewer k-steps
