@@ -982,28 +982,59 @@ int dispatch(const GroupedParams& gp, int out_dt, bool has_bias, hipStream_t st)
 //   * one of the smaller forms (gemm_tile.hip) when its tiles fit one round: the smallest that does, since a round lasts
 //     as long as one tile.  That includes every T <= G / 2 (256 x 128 tiles), and problems of up to G full tiles whose
 //     token rows are mostly padding (M = 320 is 2 x 256 rows but 3 x 128; 320 x 21 504 x 5376: 58.0 -> 44.1 us).
-//   * else full tiles in whole rounds, the last partial round cut into smaller tiles if at most half the CUs have one
-//     (T mod G <= G / 2); a fuller last round runs as full tiles.  Against a tail of four-wave 256 x 128 tiles:
-//     4100 x 5376 x 14336 255.0 -> 242.6 us (101 tiles left), 16 740 x 9216 x 3072 372.7 -> 364.1 (72 left).
+//   * else full tiles in whole rounds over either all row panels of 256 tokens or, when M is ragged, the whole ones, and
+//     one launch of smaller tiles (a tail) for what that leaves: the last partial round's tiles, and the ragged rows as
+//     the few tiles that they fill.  A tail takes the smallest form whose tiles fit one round.  Where none does, the full
+//     tiles cover all panels and the last round runs partly filled.  The cheaper of the two by split_cost.
+//     Against full tiles over all panels and a tail of four-wave 256 x 128 tiles for at most G / 2 tiles left:
+//     4100 x 5376 x 14336 255.0 -> 242.6 us (101 tiles left), 16 740 x 9216 x 3072 372.7 -> 364.1 (72 left).  With the
+//     4 ragged rows of 4100 left to the tail: an H3 MLP behind the stock fc1 (7 rounds + 112 tiles of 4 rows, instead of
+//     7.4 rounds) 826 -> 811 us.
+struct Split {
+    int panels;                // row panels that the full tiles cover
+    int full, rest;            // full tiles launched, tiles of those panels left to the tail
+    int form;                  // the tail's (TILE_FORMS: no tail)
+};
+
+// Time of a split in ns: a round of full tiles takes 1350 a k-step and 5000 for its epilogue (16 740 x 9216 x 3072: 9
+// rounds in 331 us, 4100 x 5376 x 14336: one in 162), a tail 6000 and per k-step what a full round of its form does.
+int64_t split_cost(const Split& s, int nk, int G) {
+    constexpr int kTailStep[TILE_FORMS + 1] = {180, 200, 250, 290, 420, 600, 700, 0};
+    return (int64_t)((s.full + G - 1) / G) * (1350LL * nk + 5000) +
+           (s.form < TILE_FORMS ? (int64_t)kTailStep[s.form] * nk + 6000 : 0);
+}
+
+Split split_for(const GemmParams& p, int panels, bool swiglu, int G) {
+    const int T = panels * p.tiles_n;
+    Split s{panels, (T / G) * G, T % G, TILE_FORMS};
+    // the tail's tile map takes the full-tile launch to have covered the first full / 8 positions of each per-XCD range,
+    // which holds when full is a multiple of 8 (a CU count that is a multiple of 8, as on gfx950)
+    if (s.full % 8 == 0 && (s.rest > 0 || (int64_t)panels * BM < p.M))
+        s.form = tail_form_for(p.M, p.w_rows, swiglu, panels, s.rest, G);
+    if (s.form == TILE_FORMS) s = Split{panels, T, 0, TILE_FORMS};
+    return s;
+}
+
 int launch_split(GroupedParams gp, int epi, int out_dt, bool has_bias, hipStream_t st) {
-    const GemmParams& p = gp.g[0];
-    const int T = p.tiles_m * p.tiles_n;
+    GemmParams& p = gp.g[0];
     const int G = h3host::cu_count();
+    const int nk = (p.K + BK - 1) / BK;
     const bool swiglu = epi == EPI_SWIGLU;
     const int form = tile_form_for(p.M, p.w_rows, swiglu, G);
     if (form < TILE_FORMS) return launch_tiles(p, form, out_dt, swiglu, st);
-    const int full = (T / G) * G;
-    const int rest = T - full;
-    // the tail's tile map takes the full-tile launch to have covered the first full / 8 positions of each per-XCD range,
-    // which holds when full is a multiple of 8 (a CU count that is a multiple of 8, as on gfx950); otherwise the launch
-    // keeps full tiles throughout
-    const bool tail = rest > 0 && 2 * rest <= G && full % 8 == 0;
-    gp.total_tiles = tail ? full : T;
-    const int rc = swiglu             ? dispatch<EPI_SWIGLU>(gp, H3FP8_DT_BF16, has_bias, st)
+    Split s = split_for(p, p.tiles_m, swiglu, G);
+    if (p.M % BM != 0 && p.M > BM) {
+        const Split whole = split_for(p, p.tiles_m - 1, swiglu, G);
+        if (whole.form < TILE_FORMS && split_cost(whole, nk, G) < split_cost(s, nk, G)) s = whole;
+    }
+    p.tiles_m = s.panels;
+    gp.total_tiles = s.full;
+    const int rc = s.full == 0        ? H3FP8_OK
+                   : swiglu           ? dispatch<EPI_SWIGLU>(gp, H3FP8_DT_BF16, has_bias, st)
                    : epi == EPI_PLAIN ? dispatch<EPI_PLAIN>(gp, out_dt, has_bias, st)
                                       : dispatch<EPI_AMAX>(gp, out_dt, has_bias, st);
-    if (rc || !tail) return rc;
-    return launch_tile_tail(p, full, rest, G, out_dt, swiglu, st);
+    if (rc || s.form == TILE_FORMS) return rc;
+    return launch_tile_tail(p, s.form, s.full, s.rest, out_dt, swiglu, st);
 }
 
 constexpr int64_t kMaxBufferBytes = 0x7fff0000LL;   // buffer offsets are 32-bit; keep clear of the OOB marker

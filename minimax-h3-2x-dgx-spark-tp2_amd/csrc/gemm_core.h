@@ -38,6 +38,7 @@ struct GemmParams {
     int group_m;
     int tile_offset;           // grouped launches: first block of this problem
     int tail_first;            // tail launches: the first 256 x 256 tile (in the full tiles' order) they cover; else -1
+    int tail_rest;             // ... and how many of those tiles
     int y_nt;                  // fp32 outputs: store non-temporally (the whole product is larger than the MALL)
 };
 
@@ -199,8 +200,11 @@ enum TileForm { TILE_32x64, TILE_64x64, TILE_96x64, TILE_128x64, TILE_128x128, T
 int tile_form_for(int64_t M, int64_t w_rows, bool swiglu, int64_t limit);
 // The whole problem in tiles of one form.
 int launch_tiles(GemmParams p, int form, int out_dt, bool swiglu, hipStream_t st);
-// What a launch over the first `first` 256 x 256 tiles of the problem has left (`rest` of them), each cut into the same
-// number of tiles of the smallest form that keeps all of them within `limit` workgroups.
-int launch_tile_tail(GemmParams p, int first, int rest, int limit, int out_dt, bool swiglu, hipStream_t st);
+// The tail of a launch over the first `first` 256 x 256 tiles of the first `panels` (p.tiles_m) row panels of 256 tokens:
+// the `rest` tiles that it leaves of them and the token rows past them, in tiles of one form (tail_pieces of them);
+// tail_form_for: the smallest form that keeps them within `limit` (TILE_FORMS: none).
+int64_t tail_pieces(int form, int64_t M, int64_t w_rows, int panels, int64_t rest);
+int tail_form_for(int64_t M, int64_t w_rows, bool swiglu, int panels, int64_t rest, int64_t limit);
+int launch_tile_tail(GemmParams p, int form, int first, int rest, int out_dt, bool swiglu, hipStream_t st);
 
 }  // namespace h3g

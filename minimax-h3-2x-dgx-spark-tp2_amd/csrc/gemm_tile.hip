@@ -373,17 +373,26 @@ __device__ __forceinline__ void swiglu_epilogue(const GemmParams& p, int col0, i
 
 // Workgroup -> tile of a launch that covers what a full-tile launch over the first `tail_first` tiles of the
 // XCD-contiguous map (tile_of) has left, each 256 x 256 tile cut into CW x CT tiles.  That launch took the first
-// tail_first / 8 positions of each of the 8 per-XCD ranges; the positions left are listed range by range (so consecutive
-// entries are consecutive positions), cut, and dealt out by the same XCD-contiguous rule: the pieces of a tile and
-// neighbouring tiles run on one XCD and share its L2.
-template <int CW, int CT>
+// tail_first / 8 positions of each of the 8 per-XCD ranges; the `tail_rest` positions left are listed range by range (so
+// consecutive entries are consecutive positions), cut, and dealt out by the same XCD-contiguous rule: the pieces of a tile
+// and neighbouring tiles run on one XCD and share its L2.  Behind them come the tiles of the token rows past the map's
+// tiles_m x 256, column by column.
+template <class T>
 __device__ __forceinline__ void tail_tile_of(const GemmParams& p, int id, int count, int& tm, int& tn) {
+    constexpr int CW = 256 / T::TW, CT = 256 / T::TT;
     const int xcd = id & 7, local = id >> 3;
     const int per = count >> 3, rem = count & 7;
     const int lid = (xcd < rem) ? xcd * (per + 1) + local : rem * (per + 1) + (xcd - rem) * per + local;
     int k = lid / (CW * CT);
+    if (k >= p.tail_rest) {
+        const int e = lid - p.tail_rest * (CW * CT);
+        const int rows = (p.M - p.tiles_m * 256 + T::TT - 1) / T::TT;
+        tm = p.tiles_m * CT + e % rows;
+        tn = e / rows;
+        return;
+    }
     const int sub = lid - k * (CW * CT);
-    const int T = p.tiles_m * p.tiles_n, pT = T >> 3, rT = T & 7, done = p.tail_first >> 3;
+    const int tiles = p.tiles_m * p.tiles_n, pT = tiles >> 3, rT = tiles & 7, done = p.tail_first >> 3;
     int c = 0;
     for (; c < 7; ++c) {
         const int n_c = pT + (c < rT ? 1 : 0) - done;
@@ -409,7 +418,7 @@ __global__ void __launch_bounds__(T::WAVES * 64, 2) gemm_tile_kernel(GemmParams 
     const uint32_t lds0 = lds_addr(lds);
     int tm, tn;
     if (p.tail_first >= 0) {                             // uniform
-        tail_tile_of<256 / T::TW, 256 / T::TT>(p, (int)blockIdx.x, (int)gridDim.x, tm, tn);
+        tail_tile_of<T>(p, (int)blockIdx.x, (int)gridDim.x, tm, tn);
         if (tm * T::TT >= p.M || tn * T::TC >= p.N) return;      // a piece past the edge of its 256 x 256 tile's rows
     } else {
         const int tiles_m = (p.M + T::TT - 1) / T::TT;
@@ -594,14 +603,23 @@ int launch_tiles(GemmParams p, int form, int out_dt, bool swiglu, hipStream_t st
     return launch_any(p, form, tile_count(form, p.M, p.w_rows), out_dt, swiglu, st);
 }
 
-int launch_tile_tail(GemmParams p, int first, int rest, int limit, int out_dt, bool swiglu, hipStream_t st) {
+int64_t tail_pieces(int form, int64_t M, int64_t w_rows, int panels, int64_t rest) {
+    const FormDims d = kForms[form];
+    if (256 % d.tw != 0) return INT64_MAX;
+    const int64_t edge = M - (int64_t)panels * 256;
+    return rest * (256 / d.tw) * (256 / d.tt) + (edge > 0 ? (edge + d.tt - 1) / d.tt * ((w_rows + d.tw - 1) / d.tw) : 0);
+}
+
+int tail_form_for(int64_t M, int64_t w_rows, bool swiglu, int panels, int64_t rest, int64_t limit) {
+    int f = 0;
+    while (f < TILE_FORMS && ((swiglu && !swiglu_form(f)) || tail_pieces(f, M, w_rows, panels, rest) > limit)) ++f;
+    return f;
+}
+
+int launch_tile_tail(GemmParams p, int form, int first, int rest, int out_dt, bool swiglu, hipStream_t st) {
     p.tail_first = first;
-    int f = 0, pieces = 0;
-    for (; f < TILE_FORMS; ++f) {
-        pieces = 256 / kForms[f].tw * (256 / kForms[f].tt);
-        if (256 % kForms[f].tw == 0 && !(swiglu && !swiglu_form(f)) && (int64_t)rest * pieces <= limit) break;
-    }
-    return launch_any(p, f, (int64_t)rest * pieces, out_dt, swiglu, st);
+    p.tail_rest = rest;
+    return launch_any(p, form, tail_pieces(form, p.M, p.w_rows, p.tiles_m, rest), out_dt, swiglu, st);
 }
 
 }  // namespace h3g

@@ -19,8 +19,11 @@ FORMS = ((32, 64), (64, 64), (96, 64), (128, 64), (128, 128), (192, 128), (256, 
 # the form (index of FORMS), then M, N, K
 WHOLE = [(0, 33, 16, 16), (0, 65, 528, 1040), (1, 260, 1840, 272), (2, 500, 2320, 400), (3, 700, 2320, 144),
          (4, 1000, 3008, 96), (5, 2040, 2992, 640), (6, 2300, 3312, 192), (6, 320, 21504, 256)]
-# last rounds: the form of the pieces, then M, N, K (264, 266, 286, 316, 356 full tiles)
-TAILS = [(0, 8300, 2032, 160), (1, 3400, 4800, 64), (3, 5600, 3200, 272), (4, 20200, 912, 128), (6, 22600, 1008, 400)]
+# last rounds: the form of the tail, then M, N, K, and whether the full tiles leave the ragged rows to it: 264, 266, 286,
+# 316 and 356 full tiles in all panels; 368 in the whole panels (391 in all) and 256 (272) with 4 rows past them
+TAILS = [(0, 8300, 2032, 160, False), (1, 3400, 4800, 64, False), (3, 5600, 3200, 272, False),
+         (4, 20200, 912, 128, False), (6, 22600, 1008, 400, False), (6, 4100, 5888, 272, True),
+         (0, 4100, 4096, 400, True)]
 
 
 def _count(form, M, N):
@@ -28,22 +31,24 @@ def _count(form, M, N):
     return -(-M // tt) * -(-N // tw)
 
 
-def _takes(form, M, N, tail, forms=range(len(FORMS))):
+def _takes(form, M, N, tail, forms=range(len(FORMS)), edge=False):
     G = torch.cuda.get_device_properties(0).multi_processor_count
     if not tail:
         return min((f for f in forms if _count(f, M, N) <= G), default=None) == form
-    rest = -(-M // 256) * -(-N // 256) % G
-    pieces = [(f, 256 // FORMS[f][0] * (256 // FORMS[f][1])) for f in forms if 256 % FORMS[f][0] == 0]
-    return 0 < 2 * rest <= G and min(f for f, p in pieces if rest * p <= G) == form
+    panels = M // 256 if edge else -(-M // 256)
+    rest = panels * -(-N // 256) % G
+    pieces = {f: rest * (256 // tw) * (256 // tt) + (-(-(M % 256) // tt) * -(-N // tw) if edge else 0)
+              for f, (tw, tt) in enumerate(FORMS) if f in forms and 256 % tw == 0}
+    return min((f for f, p in pieces.items() if p <= G), default=None) == form
 
 
-CASES = [(*c, False) for c in WHOLE] + [(*c, True) for c in TAILS]
+CASES = [(*c, False, False) for c in WHOLE] + [(*c[:4], True, c[4]) for c in TAILS]
 
 
-@pytest.mark.parametrize("form,M,N,K,tail", CASES)
-def test_form_equals_full_tiles(cuda, form, M, N, K, tail):
+@pytest.mark.parametrize("form,M,N,K,tail,edge", CASES)
+def test_form_equals_full_tiles(cuda, form, M, N, K, tail, edge):
     from h3_tp2_amd import ops
-    assert _takes(form, M, N, tail)
+    assert _takes(form, M, N, tail, edge=edge)
     a, w, sa, sb = serving_like(M, N, K, seed=M + K, device=cuda)
     y = ops.gemm(a, w, sa, sb)
     (ref,) = ops.grouped_gemm([(a, w, sa, sb)])
@@ -51,8 +56,8 @@ def test_form_equals_full_tiles(cuda, form, M, N, K, tail):
     assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
 
 
-@pytest.mark.parametrize("form,M,N,K,tail", CASES)
-def test_form_integer_exact_with_guards(cuda, form, M, N, K, tail):
+@pytest.mark.parametrize("form,M,N,K,tail,edge", CASES)
+def test_form_integer_exact_with_guards(cuda, form, M, N, K, tail, edge):
     from h3_tp2_amd import ops
     a, w, sa, sb = int_operands(M, N, K, seed=M + N, device=cuda)
     guard = 4096
@@ -66,8 +71,8 @@ def test_form_integer_exact_with_guards(cuda, form, M, N, K, tail):
 
 
 # one case of each form: fp16, bias, row maxima, scalar scales, strided output rows, the raw accumulator
-@pytest.mark.parametrize("form,M,N,K,tail", [c for c in CASES if c[1:3] not in ((33, 16), (320, 21504))])
-def test_form_epilogues(cuda, form, M, N, K, tail):
+@pytest.mark.parametrize("form,M,N,K,tail,edge", [c for c in CASES if c[1:3] not in ((33, 16), (320, 21504))])
+def test_form_epilogues(cuda, form, M, N, K, tail, edge):
     from h3_tp2_amd import ops
     a, w, sa, sb = int_operands(M, N, K, seed=N + K, device=cuda)
     g = torch.Generator().manual_seed(N)
@@ -91,7 +96,8 @@ def test_form_epilogues(cuda, form, M, N, K, tail):
 SWIGLU_FORMS = (1, 3, 4, 5, 6)
 SWIGLU = [(1, 1, 64, 16, False), (1, 40, 1008, 272, False), (3, 300, 2000, 400, False), (4, 600, 2000, 144, False),
           (5, 1000, 2320, 640, False), (6, 1250, 2992, 192, False),
-          (1, 2000, 4208, 128, True), (3, 5600, 1648, 272, True), (4, 20200, 496, 96, True), (6, 22600, 496, 400, True)]
+          (1, 2000, 4208, 128, True), (3, 5600, 1648, 272, True), (4, 20200, 496, 96, True), (6, 22600, 496, 400, True),
+          (6, 4100, 2944, 272, "edge"), (1, 4100, 2048, 144, "edge")]
 
 
 @pytest.mark.parametrize("form,M,F,K,tail", SWIGLU)
@@ -100,7 +106,7 @@ def test_swiglu_form_equals_oracle_of_the_accumulator(cuda, form, M, F, K, tail,
     """h and the row maxima against the oracle's SwiGLU of the kernel's own fp32 accumulator, bit for bit; some rows'
     gates are zero or far outside the compact SiLU table (those blocks take the full table), the output has guards."""
     from h3_tp2_amd import ops
-    assert _takes(form, M, 2 * F, tail, SWIGLU_FORMS)
+    assert _takes(form, M, 2 * F, tail, SWIGLU_FORMS, tail == "edge")
     a, w, sa, sb = serving_like(M, 2 * F, K, seed=M + F, device=cuda)
     sa = sa.clone()
     sa[5::37] = 0.0
