@@ -174,7 +174,14 @@ struct GlobalTables {
 __device__ __forceinline__ v4u tab16(const GlobalTables& t, int which, int c) {
     return ld16(which == 0 ? t.w : which == 1 ? t.sh : which == 2 ? t.sc : t.g, c);
 }
-// One row m processed by one wave.  OUT: bit 0 = the e4m3 row and its scale, bit 1 = the bf16 modulated row (h only:
+// What the waves of one row exchange.
+struct RowShare {
+    double ss[64];
+    float r;
+    uint32_t mx[4];
+};
+
+// One row m.  OUT: bit 0 = the e4m3 row and its scale, bit 1 = the bf16 modulated row (h only:
 // the stock producer itself).  EARLY: every table chunk is fetched together with the row (their latency overlaps the
 // row's instead of following the reduction); above 8 chunks per lane (6 for the fp32-branch form) the registers do
 // not allow it.
@@ -185,21 +192,27 @@ __device__ __forceinline__ v4u tab16(const GlobalTables& t, int which, int c) {
 // projection reading the accumulator instead of a bf16 output).
 //
 // FULL: H == 512 CPL, every chunk of every lane lies in the row (no masking of the chunks past its end).
-template <bool GATE, int OUT, int CPL, bool EARLY, bool B32, bool FULL, class MakeTables>
-__device__ __forceinline__ void rms_mod_quant_row(const RmsArgs& a, int64_t m, int lane, MakeTables tables) {
+//
+// W waves share a row, wave `part` the chunks 64 CPL part on: the sum of squares goes through the waves in order (each
+// continues its lanes' sums where the wave before left them, so the order of the additions is one wave's), the last wave
+// reduces it and hands out r, and the maxima meet in `share`.
+template <bool GATE, int OUT, int CPL, bool EARLY, bool B32, bool FULL, int W, class MakeTables>
+__device__ __forceinline__ void rms_mod_quant_row(const RmsArgs& a, int64_t m, int lane, int part, RowShare* share,
+                                                  MakeTables tables) {
+    const int c0 = lane + 64 * CPL * part;              // the lane's first chunk
     constexpr bool QUANT = (OUT & 1) != 0, WRITE_H = (OUT & 2) != 0;
     const uint32_t rb = (uint32_t)a.H * 2u;
     const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x + m * a.ldx, rb);
     v4u xv[CPL];
 #pragma unroll
-    for (int j = 0; j < CPL; ++j) xv[j] = ld16<2>(xr, lane + 64 * j);     // streamed once: non-temporal
+    for (int j = 0; j < CPL; ++j) xv[j] = ld16<2>(xr, c0 + 64 * j);     // streamed once: non-temporal
     v4u gv[GATE ? CPL : 1], bv[GATE ? CPL : 1];
     constexpr int NB = B32 ? CPL : 1;
     v4u a_lo[NB], a_hi[NB], s_lo[NB], s_hi[NB], b_e[NB];
     if (GATE && !B32) {
         const __amdgpu_buffer_rsrc_t br = make_rsrc(a.branch + m * a.ld_branch, rb);
 #pragma unroll
-        for (int j = 0; j < (GATE ? CPL : 1); ++j) bv[j] = ld16<2>(br, lane + 64 * j);
+        for (int j = 0; j < (GATE ? CPL : 1); ++j) bv[j] = ld16<2>(br, c0 + 64 * j);
     }
     if (GATE && B32) {
         const __amdgpu_buffer_rsrc_t ar = make_rsrc(a.acc + m * a.ld_acc, 2u * rb);
@@ -207,7 +220,7 @@ __device__ __forceinline__ void rms_mod_quant_row(const RmsArgs& a, int64_t m, i
         const __amdgpu_buffer_rsrc_t bsr = make_rsrc(a.bias ? a.bias : a.weight, a.bias ? rb : 0u);
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
-            const uint32_t c = (uint32_t)(lane + 64 * j);
+            const uint32_t c = (uint32_t)(c0 + 64 * j);
             a_lo[j] = __builtin_amdgcn_raw_buffer_load_b128(ar, c * 32u, 0, 2);
             a_hi[j] = __builtin_amdgcn_raw_buffer_load_b128(ar, c * 32u + 16u, 0, 2);
             s_lo[j] = __builtin_amdgcn_raw_buffer_load_b128(sr, c * 32u, 0, 0);
@@ -221,16 +234,16 @@ __device__ __forceinline__ void rms_mod_quant_row(const RmsArgs& a, int64_t m, i
     const uint32_t poison = bad ? 0x7fc07fc0u : 0u;     // OR-ed into bf16 pairs: NaN if the index is out of range
     if (GATE) {
 #pragma unroll
-        for (int j = 0; j < (GATE ? CPL : 1); ++j) gv[j] = tab16(t, 3, lane + 64 * j);
+        for (int j = 0; j < (GATE ? CPL : 1); ++j) gv[j] = tab16(t, 3, c0 + 64 * j);
     }
     constexpr int NE = EARLY ? CPL : 1;
     v4u wv_e[NE], sh_e[NE], sc_e[NE];
     if (EARLY) {
 #pragma unroll
         for (int j = 0; j < NE; ++j) {
-            wv_e[j] = tab16(t, 0, lane + 64 * j);
-            sh_e[j] = tab16(t, 1, lane + 64 * j);
-            sc_e[j] = tab16(t, 2, lane + 64 * j);
+            wv_e[j] = tab16(t, 0, c0 + 64 * j);
+            sh_e[j] = tab16(t, 1, c0 + 64 * j);
+            sc_e[j] = tab16(t, 2, c0 + 64 * j);
         }
     }
     __builtin_amdgcn_sched_barrier(0);                  // keep every load above the reduction
@@ -261,7 +274,7 @@ __device__ __forceinline__ void rms_mod_quant_row(const RmsArgs& a, int64_t m, i
         const __amdgpu_buffer_rsrc_t ro = make_rsrc(a.residual_out + m * a.ld_res, rb);
 #pragma unroll
         for (int j = 0; j < (GATE ? CPL : 1); ++j) {
-            const bool in = FULL || lane + 64 * j < nchunk;
+            const bool in = FULL || c0 + 64 * j < nchunk;
             v4u u;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
@@ -271,7 +284,7 @@ __device__ __forceinline__ void rms_mod_quant_row(const RmsArgs& a, int64_t m, i
                 u[k] = in ? (cvt_bf16x2(r0 + p0, r1 + p1) | poison) : 0u;
             }
             xv[j] = u;
-            st16(u, ro, lane + 64 * j);
+            st16(u, ro, c0 + 64 * j);
         }
     }
     // sum of squares: each square is exact in fp32, the fp64 sum rounds once to fp32 (chunks past the row add +0;
@@ -285,10 +298,26 @@ __device__ __forceinline__ void rms_mod_quant_row(const RmsArgs& a, int64_t m, i
             const float f0 = u2f(xv[j][k] << 16), f1 = u2f(xv[j][k] & 0xffff0000u);
             xf[j][2 * k] = f0;
             xf[j][2 * k + 1] = f1;
-            ss += (double)(f0 * f0);
-            ss += (double)(f1 * f1);
+            if (W == 1) {
+                ss += (double)(f0 * f0);
+                ss += (double)(f1 * f1);
+            }
         }
-    ss = wave_sum_f64(ss);
+    if (W > 1) {
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            if (part == w) {                            // wave-uniform
+                if (w > 0) ss = share->ss[lane];
+#pragma unroll
+                for (int j = 0; j < CPL; ++j)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) ss += (double)(xf[j][e] * xf[j][e]);
+                if (w < W - 1) share->ss[lane] = ss;
+            }
+            if (w < W - 1) __syncthreads();
+        }
+    }
+    if (W == 1 || part == W - 1) ss = wave_sum_f64(ss);
     const float hf = (float)a.H;
     float var = (float)ss;
     asm volatile("" : "+v"(var));                       // the division by H stays a division
@@ -296,17 +325,22 @@ __device__ __forceinline__ void rms_mod_quant_row(const RmsArgs& a, int64_t m, i
     const float d = __builtin_sqrtf(var + a.eps);     // correctly rounded (HIP's default fp32 sqrt)
     float one = 1.0f;
     asm volatile("" : "+v"(one));
-    const float r = bad ? u2f(0x7fc00000u) : one / d;  // IEEE division (torch's CPU rsqrt: 1 / sqrt)
+    float r = bad ? u2f(0x7fc00000u) : one / d;        // IEEE division (torch's CPU rsqrt: 1 / sqrt)
+    if (W > 1) {
+        if (part == W - 1 && lane == 0) share->r = r;
+        __syncthreads();
+        r = share->r;
+    }
     // modulation, bf16 rounding, row maximum (of the packed |h| pairs, two 16-bit lanes at a time; NaN patterns order
     // above +inf)
     v4u h[CPL];
     u16x2 mx2 = {0, 0};
 #pragma unroll
     for (int j = 0; j < CPL; ++j) {
-        const bool in = FULL || lane + 64 * j < nchunk;
-        const v4u wv = EARLY ? wv_e[EARLY ? j : 0] : tab16(t, 0, lane + 64 * j);
-        const v4u sh = EARLY ? sh_e[EARLY ? j : 0] : tab16(t, 1, lane + 64 * j);
-        const v4u sc = EARLY ? sc_e[EARLY ? j : 0] : tab16(t, 2, lane + 64 * j);
+        const bool in = FULL || c0 + 64 * j < nchunk;
+        const v4u wv = EARLY ? wv_e[EARLY ? j : 0] : tab16(t, 0, c0 + 64 * j);
+        const v4u sh = EARLY ? sh_e[EARLY ? j : 0] : tab16(t, 1, c0 + 64 * j);
+        const v4u sc = EARLY ? sc_e[EARLY ? j : 0] : tab16(t, 2, c0 + 64 * j);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             float o[2];
@@ -328,18 +362,24 @@ __device__ __forceinline__ void rms_mod_quant_row(const RmsArgs& a, int64_t m, i
     float s = 0.0f;
     if (QUANT) {
         mx = wave_max_u32(mx);
+        if (W > 1) {
+            if (lane == 0) share->mx[part] = mx;
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < W; ++w) mx = mx > share->mx[w] ? mx : share->mx[w];
+        }
         s = row_scale(u2f(mx));
         const float inv = inv_scale(s);
         const __amdgpu_buffer_rsrc_t qr = make_rsrc(a.q + m * a.ldq, (uint32_t)a.H);
-        if (__builtin_amdgcn_readfirstlane(mx) < 0x7f800000u) store_q<CPL, true>(h, inv, qr, lane);
-        else store_q<CPL, false>(h, inv, qr, lane);
+        if (__builtin_amdgcn_readfirstlane(mx) < 0x7f800000u) store_q<CPL, true>(h, inv, qr, c0);
+        else store_q<CPL, false>(h, inv, qr, c0);
     }
     if (WRITE_H) {
         const __amdgpu_buffer_rsrc_t hr = make_rsrc(a.h_out + m * a.ldh, rb);
 #pragma unroll
-        for (int j = 0; j < CPL; ++j) st16(h[j], hr, lane + 64 * j);
+        for (int j = 0; j < CPL; ++j) st16(h[j], hr, c0 + 64 * j);
     }
-    if (QUANT && lane == 0) a.qscale[m] = s;
+    if (QUANT && part == 0 && lane == 0) a.qscale[m] = s;
 }
 
 __device__ __forceinline__ int64_t row_index(const RmsArgs& a, int64_t m, bool& bad) {
@@ -347,6 +387,18 @@ __device__ __forceinline__ int64_t row_index(const RmsArgs& a, int64_t m, bool& 
                         : (int64_t)reinterpret_cast<const int32_t*>(a.indices)[m * a.idx_stride];
     bad = (uint64_t)i >= (uint64_t)a.n_index;
     return bad ? 0 : i;
+}
+
+// The tables of a row in global memory.
+template <bool GATE>
+__device__ __forceinline__ GlobalTables global_tables(const RmsArgs& a, int64_t i) {
+    const uint32_t rb = (uint32_t)a.H * 2u;
+    GlobalTables t;
+    t.w = make_rsrc(a.weight, rb);
+    t.sh = make_rsrc(a.shift + i * a.ld_shift, rb);
+    t.sc = make_rsrc(a.scale + i * a.ld_scale, rb);
+    t.g = make_rsrc(GATE ? a.gate + i * a.ld_gate : a.weight, rb);
+    return t;
 }
 
 // Tables read from global memory: one wave per row, 4 rows per 256-thread workgroup.
@@ -358,17 +410,30 @@ __global__ void __launch_bounds__(256) rms_mod_quant_kernel(RmsArgs a) {
     // the row's index is read first (a scalar load): its latency then overlaps the issue of the row's own loads
     bool bad0;
     const int64_t i0 = row_index(a, m, bad0);
-    rms_mod_quant_row<GATE, OUT, CPL, (CPL <= 6 || (CPL <= 8 && !B32)), B32, FULL>(a, m, lane, [&](bool& bad) {
+    rms_mod_quant_row<GATE, OUT, CPL, (CPL <= 6 || (CPL <= 8 && !B32)), B32, FULL, 1>(a, m, lane, 0, nullptr, [&](bool& bad) {
         bad = bad0;
-        const int64_t i = i0;
-        const uint32_t rb = (uint32_t)a.H * 2u;
-        GlobalTables t;
-        t.w = make_rsrc(a.weight, rb);
-        t.sh = make_rsrc(a.shift + i * a.ld_shift, rb);
-        t.sc = make_rsrc(a.scale + i * a.ld_scale, rb);
-        t.g = make_rsrc(GATE ? a.gate + i * a.ld_gate : a.weight, rb);
-        return t;
+        return global_tables<GATE>(a, i0);
     });
+}
+
+// Rows of more than 8 chunks per lane of one wave (H > 4096): four waves per row, one row per workgroup.  One wave held
+// such a row in 184 VGPRs (fp32 branch: two rows per SIMD, and 4100 rows are three rounds of 2048 of which the last has
+// four rows), its tables fetched behind the reduction; four hold it in 114-132 with the gated forms' tables fetched
+// beside it, and finish rows one by one.  H = 5376, M = 300 / 1000 / 4100 / 31 248, one wave against four: out consumer
+// 12.0 / 15.2 / 69.3 / 419 -> 7.9 / 15.5 / 49.3 / 328 us (4.6 TB/s), fc1 producer 9.5 / 11.7 / 37.8 / 215 -> 6.8 / 11.9 /
+// 34.0 / 215; two waves: 8.6 / 18.9 / 72 / 498 and 8.3 / 12.5 / 38.6 / 240.  The qkv producer (no stream of its own to
+// hide the waves' turns of the sum) only gains while its rows are few: 8.1 / 9.0 / 21.8 / 120 -> 5.4 / 7.5 / 22.0 / 135.
+template <bool GATE, int OUT, int CPL, bool B32, bool FULL>
+__global__ void __launch_bounds__(256) rms_mod_quant_wide_kernel(RmsArgs a) {
+    __shared__ RowShare share;
+    const int64_t m = blockIdx.x;
+    bool bad0;
+    const int64_t i0 = row_index(a, m, bad0);
+    rms_mod_quant_row<GATE, OUT, CPL, GATE, B32, FULL, 4>(
+        a, m, threadIdx.x & 63, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), &share, [&](bool& bad) {
+            bad = bad0;
+            return global_tables<GATE>(a, i0);
+        });
 }
 
 // The producers and the out consumer with their tables staged in LDS as fp32: one wave per row, eight rows per
@@ -640,6 +705,17 @@ int launch_rms_cpl(const RmsArgs& a, hipStream_t st) {
     return H3FP8_OK;
 }
 
+template <bool GATE, int OUT, int CPL, bool B32>
+int launch_rms_wide(const RmsArgs& a, hipStream_t st) {
+    const dim3 grid((unsigned)a.M), block(256);
+    if (a.H == 4 * 512 * CPL)
+        hipLaunchKernelGGL((rms_mod_quant_wide_kernel<GATE, OUT, CPL, B32, true>), grid, block, 0, st, a);
+    else
+        hipLaunchKernelGGL((rms_mod_quant_wide_kernel<GATE, OUT, CPL, B32, false>), grid, block, 0, st, a);
+    H3_CHECK_HIP(hipGetLastError());
+    return H3FP8_OK;
+}
+
 template <bool GATE, bool B32, int OUT, int CPL>
 int launch_rms_staged(const RmsArgs& a, hipStream_t st) {
     constexpr int rows = staged_rows<GATE>();
@@ -666,8 +742,13 @@ int launch_rms(const RmsArgs& a, hipStream_t st) {
     if (cpl <= 4) return launch_rms_cpl<GATE, OUT, 4, B32>(a, st);
     if (cpl <= 6) return launch_rms_cpl<GATE, OUT, 6, B32>(a, st);
     if (cpl <= 8) return launch_rms_cpl<GATE, OUT, 8, B32>(a, st);
-    if (cpl <= 12) return launch_rms_cpl<GATE, OUT, 12, B32>(a, st);
-    return launch_rms_cpl<GATE, OUT, 16, B32>(a, st);
+    // wider rows: four waves each, for the qkv producer up to 8 rows per CU (its one-wave form runs 12 at a time: at
+    // 1000 rows 9.0 -> 7.5 us, at 4096 20.3 -> 21.8)
+    if constexpr (!GATE) {
+        if (a.M > 8 * h3host::cu_count())
+            return cpl <= 12 ? launch_rms_cpl<GATE, OUT, 12, B32>(a, st) : launch_rms_cpl<GATE, OUT, 16, B32>(a, st);
+    }
+    return cpl <= 12 ? launch_rms_wide<GATE, OUT, 3, B32>(a, st) : launch_rms_wide<GATE, OUT, 4, B32>(a, st);
 }
 
 int check_rows(const void* p, int64_t ld, int64_t H, const char* what, const char* who) {
