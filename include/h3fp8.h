@@ -94,8 +94,8 @@ int h3fp8_gemm(const void* a, int64_t lda, const void* w, int64_t ldw, const flo
 
 /*
  * Kernel 2 + fused next-layer quant: y as h3fp8_gemm (bf16), then q [M, N] e4m3fn + scale [M] of y.
- * amax_ws: [M] fp32 workspace.  No single counterpart in the reference (its producers fuse the quant instead,
- * fp8_quant_fuse.py:23-28); the arithmetic is kernel 1's on the bf16 output.
+ * amax_ws: [M] fp32 workspace (it receives the row maxima of y).  No single counterpart in the reference (its
+ * producers fuse the quant instead, fp8_quant_fuse.py:23-28); the arithmetic is kernel 1's on the bf16 output.
  */
 int h3fp8_gemm_quant(const void* a, int64_t lda, const void* w, int64_t ldw, const float* sa, int64_t sa_stride,
                      const float* sb, int64_t sb_stride, const void* bias, void* y, int64_t ldy, int64_t M, int64_t N,
@@ -131,8 +131,8 @@ int h3fp8_gemm_swiglu(const void* a, int64_t lda, const void* w_gate_up, int64_t
                       float* row_amax, int64_t M, int64_t F, int64_t K, void* stream);
 
 /*
- * Kernel 3 with the per-token requant: h3fp8_gemm_swiglu into h_ws (bf16 [M, F], row stride F) with the row maxima in
- * amax_ws ([M] fp32), then q [M, F] e4m3fn + scale [M] (h3fp8_quant_rows_amax on h_ws).
+ * Kernel 3 with the per-token requant: h3fp8_gemm_swiglu into h_ws (bf16 [M, F], row stride F), then q [M, F] e4m3fn +
+ * scale [M] of h_ws (kernel 1's arithmetic); amax_ws ([M] fp32) receives the row maxima.
  * Replaces fp8_swiglu level 2: scale_swiglu_quant (h3_tp2/fp8_swiglu.py:191-200, kernel :72-103) after the fc1 GEMM.
  */
 int h3fp8_gemm_swiglu_quant(const void* a, int64_t lda, const void* w_gate_up, int64_t ldw, const float* sa,

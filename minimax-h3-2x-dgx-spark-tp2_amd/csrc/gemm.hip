@@ -1131,8 +1131,17 @@ int run_gemm(int epi, const uint8_t* a, int64_t lda, const uint8_t* w, int64_t l
 namespace h3host {
 int quant_rows_amax_launch(const void* x, int64_t ldx, int64_t M, int64_t K, const float* row_amax, void* q,
                            int64_t ldq, float* scale, hipStream_t st);
+int quant_rows_max_launch(const void* x, int64_t ldx, int64_t M, int64_t K, float* row_amax, void* q, int64_t ldq,
+                          float* scale, hipStream_t st);
 int quant_args_ok(const void* x, int64_t ldx, int64_t M, int64_t K, const void* q, int64_t ldq, const float* scale);
 }
+
+// Rows up to this width: the quant behind a GEMM holds its row in registers and reduces the row maxima itself (it writes
+// them to the workspace), since that costs it nothing (91 728 x 8192: 354 us, with the maxima given 353; x 3072: 124 and
+// 125) while taking them in the GEMM's epilogue costs that (kernel 3 at 91 728 x 8192 x 3072 3486 -> 3521 us, the out
+// projection 664 -> 678) and a launch to clear them.  A wider row is read twice without its maximum: there the GEMM
+// reduces it.
+constexpr int64_t kQuantOwnMax = 16384;
 
 // ---- the library-owned row-maxima buffer of h3fp8_gemm_quant_noalloc -------------------------------------------------
 // One array per device (the loader gives every device its own copy at its own address), H3FP8_NOALLOC_MAX_ROWS fp32
@@ -1189,9 +1198,11 @@ int h3fp8_gemm_quant(const void* a, int64_t lda, const void* w, int64_t ldw, con
     // the tail's arguments are checked before the GEMM is enqueued: a bad ldq leaves nothing launched
     int rc = h3host::quant_args_ok(y, ldy, M, N, q, ldq, scale);
     if (rc) return rc;
-    rc = h3fp8_gemm(a, lda, w, ldw, sa, sa_stride, sb, sb_stride, bias, y, ldy, H3FP8_DT_BF16, M, N, K, amax_ws,
-                        stream);
+    const bool own_max = N <= kQuantOwnMax;
+    rc = h3fp8_gemm(a, lda, w, ldw, sa, sa_stride, sb, sb_stride, bias, y, ldy, H3FP8_DT_BF16, M, N, K,
+                    own_max ? nullptr : amax_ws, stream);
     if (rc) return rc;
+    if (own_max) return h3host::quant_rows_max_launch(y, ldy, M, N, amax_ws, q, ldq, scale, (hipStream_t)stream);
     return h3host::quant_rows_amax_launch(y, ldy, M, N, amax_ws, q, ldq, scale, (hipStream_t)stream);
 }
 
@@ -1249,9 +1260,11 @@ int h3fp8_gemm_swiglu_quant(const void* a, int64_t lda, const void* w_gate_up, i
     H3_REQUIRE(M == 0 || (h_ws && amax_ws && q && scale), "h3fp8_gemm_swiglu_quant: null workspace or output");
     int rc = h3host::quant_args_ok(h_ws, F, M, F, q, ldq, scale);
     if (rc) return rc;
-    rc = h3fp8_gemm_swiglu(a, lda, w_gate_up, ldw, sa, sa_stride, sb, sb_stride, bias, h_ws, F, amax_ws, M, F, K,
-                               stream);
+    const bool own_max = F <= kQuantOwnMax;
+    rc = h3fp8_gemm_swiglu(a, lda, w_gate_up, ldw, sa, sa_stride, sb, sb_stride, bias, h_ws, F,
+                           own_max ? nullptr : amax_ws, M, F, K, stream);
     if (rc) return rc;
+    if (own_max) return h3host::quant_rows_max_launch(h_ws, F, M, F, amax_ws, q, ldq, scale, (hipStream_t)stream);
     return h3host::quant_rows_amax_launch(h_ws, F, M, F, amax_ws, q, ldq, scale, (hipStream_t)stream);
 }
 

@@ -195,25 +195,25 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// gemm_quant(a, w, scale_a, scale_b, bias): the plain GEMM and kernel 1 (see ops.gemm_quant)
+// gemm_quant(a, w, scale_a, scale_b, bias)
 PyObject* gemm_quant(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Operands o;
     const void* bias;
     if (n != 5 || !operands(args, false, &o) || !bias_of(args[4], o.N, at::kBFloat16, o.dev, &bias)) DECLINE;
-    at::Tensor y, q, s;
+    at::Tensor y, amax, q, s;
     int rc;
     {
         pybind11::gil_scoped_release nogil;
         y = empty(o.M, o.N, at::kBFloat16, o.dev);
+        amax = empty(o.M, 1, at::kFloat, o.dev);
         q = empty(o.M, o.N, at::kFloat8_e4m3fn, o.dev);
         s = empty(o.M, 1, at::kFloat, o.dev);
-        void* st = stream_of(o.dev);
-        rc = h3fp8_gemm(o.a->data_ptr(), o.lda, o.w->data_ptr(), o.ldw, o.sa, o.sa_stride, o.sb, o.sb_stride, bias,
-                        y.data_ptr(), o.N, H3FP8_DT_BF16, o.M, o.N, o.K, nullptr, st);
-        if (!rc) rc = h3fp8_quant_rows(y.data_ptr(), o.N, o.M, o.N, q.data_ptr(), o.N, static_cast<float*>(s.data_ptr()), st);
+        rc = h3fp8_gemm_quant(o.a->data_ptr(), o.lda, o.w->data_ptr(), o.ldw, o.sa, o.sa_stride, o.sb, o.sb_stride, bias,
+                              y.data_ptr(), o.N, o.M, o.N, o.K, static_cast<float*>(amax.data_ptr()), q.data_ptr(), o.N,
+                              static_cast<float*>(s.data_ptr()), stream_of(o.dev));
     }
-    if (rc) return failed("h3fp8_gemm", rc);
+    if (rc) return failed("h3fp8_gemm_quant", rc);
     return tuple_of(std::move(y), std::move(q), std::move(s));
     END_HANDLE_TH_ERRORS
 }
@@ -225,19 +225,19 @@ PyObject* gemm_swiglu_quant(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const void* bias;
     if (n != 5 || !operands(args, false, &o) || o.N % 2 || !bias_of(args[4], o.N, at::kBFloat16, o.dev, &bias)) DECLINE;
     const int64_t F = o.N / 2;
-    at::Tensor h, q, s;
+    at::Tensor h, amax, q, s;
     int rc;
     {
         pybind11::gil_scoped_release nogil;
         h = empty(o.M, F, at::kBFloat16, o.dev);
+        amax = empty(o.M, 1, at::kFloat, o.dev);
         q = empty(o.M, F, at::kFloat8_e4m3fn, o.dev);
         s = empty(o.M, 1, at::kFloat, o.dev);
-        void* st = stream_of(o.dev);
-        rc = h3fp8_gemm_swiglu(o.a->data_ptr(), o.lda, o.w->data_ptr(), o.ldw, o.sa, o.sa_stride, o.sb, o.sb_stride, bias,
-                               h.data_ptr(), F, nullptr, o.M, F, o.K, st);
-        if (!rc) rc = h3fp8_quant_rows(h.data_ptr(), F, o.M, F, q.data_ptr(), F, static_cast<float*>(s.data_ptr()), st);
+        rc = h3fp8_gemm_swiglu_quant(o.a->data_ptr(), o.lda, o.w->data_ptr(), o.ldw, o.sa, o.sa_stride, o.sb, o.sb_stride,
+                                     bias, o.M, F, o.K, h.data_ptr(), static_cast<float*>(amax.data_ptr()), q.data_ptr(),
+                                     F, static_cast<float*>(s.data_ptr()), stream_of(o.dev));
     }
-    if (rc) return failed("h3fp8_gemm_swiglu", rc);
+    if (rc) return failed("h3fp8_gemm_swiglu_quant", rc);
     return tuple_of(std::move(q), std::move(s));
     END_HANDLE_TH_ERRORS
 }

@@ -61,13 +61,14 @@ __device__ __forceinline__ uint2 chunk_quant(uint4 v, float inv) {
 // WPR waves per row, CPL 16-byte chunks per lane held in registers: wave p of a row owns its chunks
 // 64 CPL p .. 64 CPL (p + 1) - 1.  KNOWN_AMAX: the row maximum comes from row_amax (fp32 bits) instead of the row, so
 // the waves of a row are independent; otherwise two waves of a row exchange their maxima through LDS (one barrier),
-// and no wave leaves before it: a wave of a row at or past M reads and writes nothing (empty buffer ranges).
+// and no wave leaves before it: a wave of a row at or past M reads and writes nothing (empty buffer ranges).  Without
+// KNOWN_AMAX the maxima are written to row_amax if it is given.
 // STORE_AUX: the cache policy of the code stores (the launcher's choice, below).
 template <int CPL, bool KNOWN_AMAX, int WPR = 1, int STORE_AUX = 16>
 __global__ void __launch_bounds__(256) quant_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_t M,
                                                          int64_t K, uint8_t* __restrict__ q, int64_t ldq,
                                                          float* __restrict__ scale,
-                                                         const float* __restrict__ row_amax) {
+                                                         float* __restrict__ row_amax) {
     static_assert(WPR == 1 || WPR == 2, "one or two waves per row");
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t row = (int64_t)blockIdx.x * (4 / WPR) + wave / WPR;
@@ -121,7 +122,10 @@ __global__ void __launch_bounds__(256) quant_rows_kernel(const uint16_t* __restr
             __builtin_amdgcn_raw_buffer_store_b64(v2u{o.x, o.y}, qr, (uint32_t)(lane + 64 * j) * 8u, 0, STORE_AUX);
         }
     }
-    if (live && lane == 0) scale[row] = s;
+    if (live && lane == 0) {
+        scale[row] = s;
+        if (!KNOWN_AMAX && row_amax) row_amax[row] = amax;
+    }
 }
 
 // Rows too wide for the register-resident form: the row is read twice (max pass, then quant pass).
@@ -129,7 +133,7 @@ template <bool KNOWN_AMAX>
 __global__ void __launch_bounds__(256) quant_rows_wide_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_t M,
                                                               int64_t K, uint8_t* __restrict__ q, int64_t ldq,
                                                               float* __restrict__ scale,
-                                                              const float* __restrict__ row_amax) {
+                                                              float* __restrict__ row_amax) {
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= M) return;
@@ -150,12 +154,15 @@ __global__ void __launch_bounds__(256) quant_rows_wide_kernel(const uint16_t* __
     const float inv = inv_scale(s);
     uint2* qr = reinterpret_cast<uint2*>(q + row * ldq);
     for (int64_t c = lane; c < nchunk; c += 64) qr[c] = chunk_quant<false>(xr[c], inv);
-    if (lane == 0) scale[row] = s;
+    if (lane == 0) {
+        scale[row] = s;
+        if (!KNOWN_AMAX && row_amax) row_amax[row] = amax;
+    }
 }
 
 template <bool KNOWN>
 int launch_quant(const void* x, int64_t ldx, int64_t M, int64_t K, void* q, int64_t ldq, float* scale,
-                 const float* row_amax, hipStream_t st) {
+                 float* row_amax, hipStream_t st) {
     if (M == 0) return H3FP8_OK;
     const int64_t nchunk = K >> 3;
     const int64_t cpl = (nchunk + 63) / 64;
@@ -284,7 +291,14 @@ int quant_rows_amax_launch(const void* x, int64_t ldx, int64_t M, int64_t K, con
                            int64_t ldq, float* scale, hipStream_t st) {
     int rc = check_quant_args(x, ldx, M, K, q, ldq, scale);
     if (rc) return rc;
-    return launch_quant<true>(x, ldx, M, K, q, ldq, scale, row_amax, st);
+    return launch_quant<true>(x, ldx, M, K, q, ldq, scale, const_cast<float*>(row_amax), st);   // only read
+}
+
+int quant_rows_max_launch(const void* x, int64_t ldx, int64_t M, int64_t K, float* row_amax, void* q, int64_t ldq,
+                          float* scale, hipStream_t st) {
+    int rc = check_quant_args(x, ldx, M, K, q, ldq, scale);
+    if (rc) return rc;
+    return launch_quant<false>(x, ldx, M, K, q, ldq, scale, row_amax, st);
 }
 }  // namespace h3host
 

@@ -267,11 +267,7 @@ def scaled_mm(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor, scale_b: 
 
 def gemm_quant(a: torch.Tensor, w: torch.Tensor, scale_a: torch.Tensor, scale_b: torch.Tensor,
                bias: torch.Tensor | None = None):
-    """GEMM to bf16 y plus the per-token e4m3 quant of y: returns (y bf16 [M, N], q e4m3fn [M, N], scale fp32 [M, 1]).
-
-    The quant reduces the row maxima itself: it holds its row in registers, so they cost it nothing (91 728 x 3072:
-    124 us, with the maxima given 125), while taking them in the GEMM's epilogue costs that (out projection of 91 728
-    rows 664 -> 678 us) and a launch to clear them."""
+    """GEMM to bf16 y plus the per-token e4m3 quant of y: returns (y bf16 [M, N], q e4m3fn [M, N], scale fp32 [M, 1])."""
     if _host is not None and (out := _host.gemm_quant(a, w, scale_a, scale_b, bias)) is not None:
         return out
     N = w.shape[0]
@@ -279,12 +275,12 @@ def gemm_quant(a: torch.Tensor, w: torch.Tensor, scale_a: torch.Tensor, scale_b:
     _check_bias(bias, N, a.device)
     dev = a.device
     y = torch.empty((M, N), device=dev, dtype=torch.bfloat16)
+    amax = torch.empty((M,), device=dev, dtype=torch.float32)
     q = torch.empty((M, N), device=dev, dtype=E4M3)
     s = torch.empty((M, 1), device=dev, dtype=torch.float32)
-    _lib.call("h3fp8_gemm", a.data_ptr(), _rows(a, "a"), w.data_ptr(), _rows(w, "w"), sa.data_ptr(), sa_st,
-              sb.data_ptr(), sb_st, bias.data_ptr() if bias is not None else None, y.data_ptr(), N,
-              _DT[torch.bfloat16], M, N, a.shape[1], None, _stream(a))
-    _lib.call("h3fp8_quant_rows", y.data_ptr(), N, M, N, q.data_ptr(), N, s.data_ptr(), _stream(a))
+    _lib.call("h3fp8_gemm_quant", a.data_ptr(), _rows(a, "a"), w.data_ptr(), _rows(w, "w"), sa.data_ptr(), sa_st,
+              sb.data_ptr(), sb_st, bias.data_ptr() if bias is not None else None, y.data_ptr(), N, M, N, a.shape[1],
+              amax.data_ptr(), q.data_ptr(), N, s.data_ptr(), _stream(a))
     return y, q, s
 
 
@@ -325,9 +321,7 @@ def gemm_swiglu(a: torch.Tensor, w_gate_up: torch.Tensor, scale_a: torch.Tensor,
 
 def gemm_swiglu_quant(a: torch.Tensor, w_gate_up: torch.Tensor, scale_a: torch.Tensor, scale_b: torch.Tensor,
                       bias: torch.Tensor | None = None, h_ws: torch.Tensor | None = None):
-    """fc1 + SwiGLU + per-token requant (fp8_swiglu level 2, h3_tp2/fp8_swiglu.py:191-200): (q [M, F], scale [M, 1]).
-    The requant reduces the row maxima of h itself, as in ``gemm_quant`` (91 728 x 8192 behind 3072: kernel 3 3486 us,
-    with the maxima 3521; the quant 354 us, with the maxima given 353)."""
+    """fc1 + SwiGLU + per-token requant (fp8_swiglu level 2, h3_tp2/fp8_swiglu.py:191-200): (q [M, F], scale [M, 1])."""
     if _host is not None and h_ws is None:
         out = _host.gemm_swiglu_quant(a, w_gate_up, scale_a, scale_b, bias)
         if out is not None:
@@ -339,12 +333,12 @@ def gemm_swiglu_quant(a: torch.Tensor, w_gate_up: torch.Tensor, scale_a: torch.T
     if h_ws is None:
         h_ws = torch.empty((M, F), device=dev, dtype=torch.bfloat16)
     check_buffer(h_ws, "h_ws", (M, F), torch.bfloat16, dev, contiguous=True)   # the C side writes rows of F
+    amax = torch.empty((M,), device=dev, dtype=torch.float32)
     q = torch.empty((M, F), device=dev, dtype=E4M3)
     s = torch.empty((M, 1), device=dev, dtype=torch.float32)
-    _lib.call("h3fp8_gemm_swiglu", a.data_ptr(), _rows(a, "a"), w_gate_up.data_ptr(), _rows(w_gate_up, "w"),
-              sa.data_ptr(), sa_st, sb.data_ptr(), sb_st, bias.data_ptr() if bias is not None else None,
-              h_ws.data_ptr(), F, None, M, F, a.shape[1], _stream(a))
-    _lib.call("h3fp8_quant_rows", h_ws.data_ptr(), F, M, F, q.data_ptr(), F, s.data_ptr(), _stream(a))
+    _lib.call("h3fp8_gemm_swiglu_quant", a.data_ptr(), _rows(a, "a"), w_gate_up.data_ptr(), _rows(w_gate_up, "w"),
+              sa.data_ptr(), sa_st, sb.data_ptr(), sb_st, bias.data_ptr() if bias is not None else None, M, F,
+              a.shape[1], h_ws.data_ptr(), amax.data_ptr(), q.data_ptr(), F, s.data_ptr(), _stream(a))
     return q, s
 
 
