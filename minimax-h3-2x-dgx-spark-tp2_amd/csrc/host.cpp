@@ -19,12 +19,15 @@
 
 namespace {
 
+constexpr c10::DispatchKeySet kWrappers({c10::DispatchKey::Functionalize, c10::DispatchKey::FuncTorchGradWrapper,
+                                         c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::Batched});
+
 // A plain GPU tensor with memory of its own (no subclass, no wrapper of a function transform).
 const at::Tensor* plain(PyObject* o) {
     if (!THPVariable_CheckExact(o)) return nullptr;
     const at::Tensor& t = THPVariable_Unpack(o);
     if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || !t.has_storage() ||
-        t.unsafeGetTensorImpl()->is_python_dispatch())
+        t.unsafeGetTensorImpl()->is_python_dispatch() || t.key_set().has_any(kWrappers))
         return nullptr;
     return &t;
 }

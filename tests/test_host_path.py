@@ -129,3 +129,13 @@ def test_runs_on_the_current_stream_and_under_capture(cuda):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, ref) and torch.equal(s, s_ref) and torch.equal(q.view(torch.uint8), q_ref.view(torch.uint8))
+
+
+@pytest.mark.gpu
+def test_function_transforms_stay_on_the_python_path(cuda, monkeypatch):
+    x = torch.randn(2, 4, 64, device=cuda).to(BF16)
+    _both(monkeypatch, lambda: torch.func.vmap(ops.quant_rows)(x))
+    _both(monkeypatch, lambda: torch.func.functionalize(ops.silu_mul_quant)(x[0]))
+    _both(monkeypatch, lambda: ops.quant_rows(x[0].clone().requires_grad_()))
+    with torch.inference_mode():
+        _both(monkeypatch, lambda: ops.quant_rows(x[0]))
