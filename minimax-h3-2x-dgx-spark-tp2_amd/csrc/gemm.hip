@@ -997,7 +997,9 @@ struct Split {
 };
 
 // Time of a split in ns: a round of full tiles takes 1350 a k-step and 5000 for its epilogue (16 740 x 9216 x 3072: 9
-// rounds in 331 us, 4100 x 5376 x 14336: one in 162), a tail 6000 and per k-step what a full round of its form does.
+// rounds in 343 us; 4100 x 5376 x 7168: one in 86), a tail 6000 and per k-step what a full round of its form does
+// (measured: 101 tiles as 202 of 256 x 128, 56 k-steps, 44 us; 112 x 4 rows as 224 of 128 x 64, 42 k-steps, 25-27 us,
+// with their weights from HBM).
 int64_t split_cost(const Split& s, int nk, int G) {
     constexpr int kTailStep[TILE_FORMS + 1] = {180, 200, 250, 290, 420, 600, 700, 0};
     return (int64_t)((s.full + G - 1) / G) * (1350LL * nk + 5000) +

@@ -1,19 +1,20 @@
 // Kernel 2's forms of smaller tiles (gfx950): problems and last rounds that 256 x 256 tiles would run on a few CUs.
 //
 // One workgroup computes one tile, TW weight rows x TT token rows, with WN x WM waves of NI x NJ MFMA blocks each, and
-// the launch has at most one tile per CU, so the time is that of one tile: the form taken is the smallest whose tiles fit.  Every output element goes through the same MFMA sequence and
-// epilogue arithmetic as in the 256 x 256 tiles (v_mfma 32x32x64, weight row at A-row n % 32, token at B-column m % 32,
-// k ascending from a zero accumulator), so the output is bitwise the same.
+// the launch has at most one tile per CU, so the time is that of one tile: the form taken is the smallest whose tiles
+// fit.  Every output element goes through the same MFMA sequence and epilogue arithmetic as in the 256 x 256 tiles
+// (v_mfma 32x32x64, weight row at A-row n % 32, token at B-column m % 32, k ascending from a zero accumulator), so the
+// output is bitwise the same.
 //
 // What bounds it: a k-step loads (TW + TT) x 128 bytes per CU by LDS-DMA, 16 cycles per 1 KiB instruction at best (64
-// bytes per cycle and CU; measured 20 with out-of-range loads, 25-30 with real ones, where L2 misses wait on the MALL or
-// HBM), while its MFMAs take TW TT / 32 cycles.  The small tiles are bound by those loads and by the
-// latency of a k-step (barrier, fragment reads, MFMAs), so they keep 7-8 k-steps in flight in an LDS ring and take one
-// barrier per two k-steps; the large ones are bound by the fragment reads of their waves (LDS returns 95 bytes per cycle
-// to one wave per SIMD, 250 to two), so they run two waves per SIMD.  Measured against the forms before (128 x 192 and
-// 256 x 128 tiles of four waves), M x N x K, operands in the MALL: 64 x 5376 x 14336 71.0 -> 20.9 us, 200 x 5376 x 14336
-// 69.6 -> 29.2, 512 x 6144 x 4096 24.6 -> 16.9, 2048 x 3072 x 3072 23.5 -> 22.0, 1000 x 5376 x 14336 81.8 -> 67.5,
-// 768 x 9216 x 3072 32.8 -> 26.9, 1300 x 5376 x 7168 60.7 -> 49.5.
+// bytes per cycle and CU; measured 20 with out-of-range loads, 25-30 with real ones, where L2 misses wait on the MALL
+// or HBM), while its MFMAs take TW TT / 32 cycles.  The small tiles are bound by those loads and by the latency of a
+// k-step (barrier, fragment reads, MFMAs), so they keep 7-8 k-steps in flight in an LDS ring and take one barrier per
+// two k-steps; the large ones are bound by the fragment reads of their waves (LDS returns 95 bytes per cycle to one
+// wave per SIMD, 250 to two), so they run two waves per SIMD.  Measured against the forms before (128 x 192 and 256 x
+// 128 tiles of four waves), M x N x K, operands in the MALL: 64 x 5376 x 14336 71.0 -> 20.9 us, 200 x 5376 x 14336 69.6
+// -> 29.2, 512 x 6144 x 4096 24.6 -> 16.9, 2048 x 3072 x 3072 23.5 -> 21.4, 1000 x 5376 x 14336 81.8 -> 67.5, 768 x
+// 9216 x 3072 28.9 -> 23.2.
 #include "gemm_core.h"
 
 namespace {
