@@ -107,9 +107,10 @@ __device__ __forceinline__ v4u buffer_desc(const void* base, uint32_t bytes) {
 // 16 bytes per lane from a buffer straight into LDS at lds_base + 16 * lane (buffer_load_dwordx4 ... lds).
 // Written as inline asm so that the compiler's wait-count pass does not track these loads: it cannot tell one LDS
 // stage from another and would wait for every in-flight load before each LDS read.  The kernel therefore places
-// every wait on these loads itself (wait_vm before the barrier that publishes a stage).
+// every wait on these loads itself (wait_vm before the barrier that publishes a stage).  The s_nop is the wait state that
+// gfx9 needs between a scalar write of M0 and an LDS-DMA load, which the compiler leaves out of inline asm.
 __device__ __forceinline__ void dma16(v4u desc, uint32_t lds_base, uint32_t voff) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                  :
                  : "s"(lds_base), "v"(voff), "s"(desc)
                  : "memory", "m0");
@@ -117,7 +118,7 @@ __device__ __forceinline__ void dma16(v4u desc, uint32_t lds_base, uint32_t voff
 
 // The same load at a further uniform byte offset.
 __device__ __forceinline__ void dma16_at(v4u desc, uint32_t lds_base, uint32_t voff, uint32_t soff) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :
                  : "s"(lds_base), "v"(voff), "s"(desc), "s"(soff)
                  : "memory", "m0");
@@ -125,7 +126,7 @@ __device__ __forceinline__ void dma16_at(v4u desc, uint32_t lds_base, uint32_t v
 
 // ... with the non-temporal hint, for operands that stream through once.
 __device__ __forceinline__ void dma16_at_nt(v4u desc, uint32_t lds_base, uint32_t voff, uint32_t soff) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
                  :
                  : "s"(lds_base), "v"(voff), "s"(desc), "s"(soff)
                  : "memory", "m0");
@@ -138,7 +139,7 @@ __device__ __forceinline__ uint32_t lds_addr(const uint8_t* p) {
 
 // 4 bytes per lane straight into LDS at lds_base + 4 * lane (buffer_load_dword ... lds); untracked like dma16.
 __device__ __forceinline__ void dma4(v4u desc, uint32_t lds_base, uint32_t voff) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
                  :
                  : "s"(lds_base), "v"(voff), "s"(desc)
                  : "memory", "m0");
