@@ -367,7 +367,7 @@ __device__ __forceinline__ void kstep(uint8_t* lds, uint32_t lds0, int g, const 
 // Scales come from the tile's scale set in LDS (loaded with the tile's first k-step).
 template <int OUT_DT, bool HAS_BIAS, int EPI>
 __device__ __forceinline__ void epilogue(const GemmParams& p, int tm, int tn, uint8_t* lds, int set, int wave, int wn,
-                                         int wm, int lane, v16f acc[4][4]) {
+                                         int wm, int lane, v16f (&acc)[4][4]) {
     constexpr int NI = 4;                               // MFMA tiles along the channels per wave
     const int wcol = tn * BN + wn * 128;                // the wave's first output channel
     const int wsb = wn * 128;                           // ... and its first entry in the tile's sb set
@@ -720,6 +720,7 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(GroupedParams gp) {
         // the tile's last k-step publishes the next k-step's stage but leaves its fragment registers free for the
         // epilogue; they are read after it
         kstep<EPI, false, false>(lds, lds0, g, I, wofs, wn, wm, lane, acc, fa0, fb0, fa1, fb1);
+        accumulators_ready<true>(acc);
         if (I.valid) cursor_next<EPI, GROUPED>(I, gp, lds0, wave, lane);
         ++g;
         epilogue<OUT_DT, HAS_BIAS, EPI>(p, tm, tn, lds, c % NSCALE, wave, wn, wm, lane, acc);
@@ -834,7 +835,8 @@ __global__ void __launch_bounds__(64) gemm_rows_kernel(GemmParams p) {
     };
     auto next = [](uint32_t slot) { return slot == (ROWS_DEPTH - 1) * ROWS_STAGE ? 0u : slot + ROWS_STAGE; };
 
-    v16f acc;
+    v16f blk[1][1];
+    v16f& acc = blk[0][0];
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.f;
 #pragma unroll
@@ -867,6 +869,7 @@ __global__ void __launch_bounds__(64) gemm_rows_kernel(GemmParams p) {
         kstep(F, G);
         kstep(G, F);
     }
+    accumulators_ready<true>(blk);
     wait_vm0();                                         // the out-of-range tail loads have landed before the exit
     wait_lgkm0();
 

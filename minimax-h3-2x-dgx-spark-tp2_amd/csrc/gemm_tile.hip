@@ -491,10 +491,7 @@ __global__ void __launch_bounds__(T::WAVES * 64, 2) gemm_tile_kernel(GemmParams 
         tile_kstep<T, true, true, true>(lds, lds0, rd, ld, L, wave, wn, wm, lane, acc, F, G);
     }
     tile_kstep<T, false, false, false>(lds, lds0, rd, ld, L, wave, wn, wm, lane, acc, G, F);
-    // An accumulator is read no sooner than 32 wait states after its last MFMA: at the 19 that the compiler leaves, copies
-    // of the last block's last registers have come out without that MFMA's sum.
-    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
+    accumulators_ready<(T::WAVES <= 4)>(acc);
     // the reads of the last k-steps have returned before the ring is reused
     wait_lgkm0();
     // the ring becomes the epilogue's staging area once every wave's last reads have returned and the trailing

@@ -1,6 +1,8 @@
-"""Wait states that gfx950 needs from the program and that the compiler does not put around inline asm, checked in the
-listing of every kernel of the built library:
+"""Wait states that gfx950 needs from the program, checked in the listing of every kernel of the built library: around inline
+asm the compiler puts none.
 
+* an accumulator is read, copied or overwritten no sooner than 24 wait states behind the MFMA that wrote it (v_mfma
+  32x32x64 on 8-bit operands needs 20; 24 is what the kernels put there, so a smaller gap has come in before them);
 * an LDS-DMA load (buffer_load ... lds) comes at least one wait state behind the scalar instruction that wrote M0, its LDS
   address;
 * a memory instruction reads scalar registers that a vector instruction wrote at least five wait states before.
@@ -17,6 +19,7 @@ import pytest
 from h3_tp2_amd import _lib
 
 OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+MFMA_STATES = 24
 M0_STATES = 1
 SGPR_STATES = 5
 
@@ -84,6 +87,41 @@ def _within(insns, i, states):
         todo += [(n, gap + _states(*insns[j][:2])) for n in _next(insns, j)]
 
 
+def _vregs(text):
+    out = {(c, int(i)) for c, i in re.findall(r"\b([av])(\d+)\b", text)}
+    for c, lo, hi in re.findall(r"\b([av])\[(\d+):(\d+)\]", text):
+        out |= {(c, i) for i in range(int(lo), int(hi) + 1)}
+    return out
+
+
+def mfma_gaps(insns):
+    """(wait states, MFMA, reader) of every access too close behind the MFMA that wrote its register."""
+    regs = [None] * len(insns)
+    out = []
+    for i, (op, args, _) in enumerate(insns):
+        if not op.startswith("v_mfma"):
+            continue
+        todo, seen = [(n, 0, frozenset(_vregs(args.split(", ")[0]))) for n in _next(insns, i)], {}
+        while todo:
+            j, gap, dest = todo.pop()
+            if gap >= MFMA_STATES or not dest or seen.get((j, dest), MFMA_STATES) <= gap:
+                continue
+            seen[(j, dest)] = gap
+            o, a, _ = insns[j]
+            if o.startswith("v_mfma"):                    # its own accumulator is forwarded; the other operands are not
+                d, x, y = a.split(", ")[:3]
+                if dest & _vregs(x + " " + y):
+                    out.append((gap, i, j))
+                dest = dest - _vregs(d)
+            else:
+                regs[j] = _vregs(a) if regs[j] is None else regs[j]
+                if dest & regs[j]:
+                    out.append((gap, i, j))
+                    continue
+            todo += [(n, gap + _states(o, a), dest) for n in _next(insns, j)]
+    return out
+
+
 def m0_gaps(insns):
     """The LDS-DMA loads too close behind a write of M0."""
     return [j for i, (op, args, _) in enumerate(insns) if op.startswith("s_") and re.match(r"m0\b", args)
@@ -123,6 +161,11 @@ def kernels(tmp_path_factory):
     return out
 
 
+def test_accumulators_are_read_late_enough(kernels):
+    bad = {k: min(g) for k, g in ((k, mfma_gaps(ins)) for k, ins in kernels.items()) if g}
+    assert not bad, bad
+
+
 def test_m0_is_written_early_enough(kernels):
     bad = {k: len(g) for k, g in ((k, m0_gaps(ins)) for k, ins in kernels.items()) if g}
     assert not bad, bad
@@ -147,6 +190,16 @@ def _insns(*lines):
 
 
 _LOAD = "buffer_load_dwordx4 v1, s[4:7], 0 offen lds"
+
+
+def test_finds_a_copy_close_behind_its_mfma():
+    mfma, copy = "v_mfma_f32_32x32x64_f8f6f4 a[0:15], v[0:7], v[8:15], a[0:15]", "v_accvgpr_read_b32 v20, a15"
+    assert mfma_gaps(_insns(mfma, "s_nop 15", "s_nop 6", copy)) == [(23, 0, 3)]
+    assert mfma_gaps(_insns(mfma, "s_nop 15", "s_nop 7", copy)) == []
+    # the next MFMA takes the block over, and what follows counts from it
+    assert mfma_gaps(_insns(mfma, "s_nop 15", mfma, "s_nop 15", "s_nop 6", copy)) == [(23, 2, 5)]
+    # a loop's exit is far enough, its way back to the top is not
+    assert mfma_gaps(_insns(copy, mfma, ("s_cbranch_scc1 65533", 0), "s_nop 15", "s_nop 6", copy)) == [(1, 1, 0)]
 
 
 def test_finds_a_load_right_behind_m0():
