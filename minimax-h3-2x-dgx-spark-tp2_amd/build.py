@@ -1,5 +1,5 @@
-"""Build libh3fp8.so (the HIP kernels + C ABI) for gfx950 with hipcc, and _host.so (the native host path of the common
-calls, a CPython extension on the installed torch) with g++, in-tree.
+"""Build libh3fp8.so (the HIP kernels + C ABI) for gfx950 with hipcc, and _host (the native host path of the common calls, a
+CPython extension on the installed torch) with g++, in-tree.
 
     python minimax-h3-2x-dgx-spark-tp2_amd/build.py [--jobs N] [--asm]
 
@@ -15,12 +15,13 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "h3_tp2_amd", "libh3fp8.so")
-HOST = os.path.join(HERE, "h3_tp2_amd", "_host.so")
+HOST = os.path.join(HERE, "h3_tp2_amd", "_host" + sysconfig.get_config_var("EXT_SUFFIX"))
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 
 ARCH = "gfx950"
@@ -52,9 +53,7 @@ def _compile(src: str, asm: bool) -> str:
 
 
 def build_host() -> str:
-    """_host.so: csrc/host.cpp against torch's headers, linked to libh3fp8.so next to it."""
-    import sysconfig
-
+    """_host: csrc/host.cpp against torch's headers, linked to libh3fp8.so next to it."""
     import torch
     from torch.utils import cpp_extension
     root = os.environ.get("ROCM_PATH", "/opt/rocm")
@@ -62,6 +61,7 @@ def build_host() -> str:
     lib_dir = os.path.join(os.path.dirname(torch.__file__), "lib")
     tmp = HOST + ".tmp"
     subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+                    f'-DH3_TORCH_VERSION="{torch.__version__}"',
                     f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{d}" for d in includes),
                     os.path.join(CSRC, "host.cpp"), "-o", tmp, f"-L{os.path.dirname(LIB)}", "-lh3fp8", f"-L{lib_dir}",
                     "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", "-Wl,-rpath,$ORIGIN"], check=True)
@@ -77,9 +77,16 @@ def build(jobs: int = 4, asm: bool = False, verbose: bool = True) -> str:
     tmp = LIB + ".tmp"
     subprocess.run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs], check=True)
     os.replace(tmp, LIB)
-    build_host()
     if verbose:
         print(f"built {LIB} from {len(srcs)} sources", file=sys.stderr)
+    try:
+        build_host()
+        if verbose:
+            print(f"built {HOST}", file=sys.stderr)
+    except (subprocess.CalledProcessError, OSError, ImportError) as e:      # no g++, no torch headers: Python does its work
+        if os.path.exists(HOST):
+            os.remove(HOST)                               # of an earlier library
+        print(f"the library is built, {HOST} is not ({e}): its calls take the Python path", file=sys.stderr)
     return LIB
 
 

@@ -368,5 +368,15 @@ PyMODINIT_FUNC PyInit__host() {
         PyErr_Format(PyExc_ImportError, "libh3fp8 ABI version %d, expected %d", h3fp8_abi_version(), H3FP8_ABI_VERSION);
         return nullptr;
     }
-    return PyModule_Create(&kModule);
+    // torch's C++ interface is that of one version
+    PyObject* torch = PyImport_ImportModule("torch");
+    PyObject* version = torch ? PyObject_GetAttrString(torch, "__version__") : nullptr;
+    PyObject* text = version ? PyObject_Str(version) : nullptr;
+    Py_XDECREF(torch);
+    Py_XDECREF(version);
+    if (!text) return nullptr;
+    const bool same = PyUnicode_CompareWithASCIIString(text, H3_TORCH_VERSION) == 0;
+    if (!same) PyErr_Format(PyExc_ImportError, "built on torch %s, loaded by torch %U", H3_TORCH_VERSION, text);
+    Py_DECREF(text);
+    return same ? PyModule_Create(&kModule) : nullptr;
 }

@@ -6,12 +6,16 @@ if the library is missing or fails to load, every call raises -- the product pat
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import logging
 import os
 import threading
 
+logger = logging.getLogger("h3_tp2_amd")
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libh3fp8.so")
-HOST_PATH = os.path.join(_HERE, "_host.so")
+HOST_PATH = os.path.join(_HERE, "_host" + importlib.machinery.EXTENSION_SUFFIXES[0])   # of this interpreter
 ABI_VERSION = 1
 
 H3FP8_DT_BF16 = 0
@@ -119,9 +123,14 @@ def call(name: str, *args) -> None:
 
 
 def host():  # noqa: ANN201
-    """The native host path of the common calls (csrc/host.cpp), or None where it or the library is not built: every
-    call then takes the Python path to the same kernels, and raises there if the library is missing."""
+    """The native host path of the common calls (csrc/host.cpp), or None where it or the library is not built or does not
+    load (built on another torch): every call then takes the Python path to the same kernels, and raises there if the
+    library is missing."""
     if not (os.path.exists(HOST_PATH) and os.path.exists(LIB_PATH)):
         return None
-    from . import _host
+    try:
+        from . import _host
+    except ImportError as e:
+        logger.warning("the native host path does not load, its calls take the Python path: %s", e)
+        return None
     return _host

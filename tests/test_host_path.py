@@ -1,5 +1,10 @@
 """The native host path of the common calls (csrc/host.cpp) against the Python path of the same functions: the same
 outputs for every form it takes, and every other form left to the Python path -- taken or refused with the same error."""
+import os
+import shutil
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -26,6 +31,26 @@ def test_leaves_cpu_tensors_subclasses_and_other_arguments_to_python():
         assert h.rms_quant(bad, x, x, x, s, 1e-6) is None and h.gate_rms_quant(bad, x, x, x, x, x, s, 1e-6) is None
     for f in (h.quant_rows, h.gemm, h.scaled_mm, h.gemm_quant, h.gemm_swiglu_quant, h.rms_quant, h.gate_rms_quant):
         assert f() is None
+
+
+# A package whose native part cannot be loaded, or belongs to another torch, imports and keeps the Python path.
+@pytest.mark.parametrize("how", ["not a library", "another torch"])
+def test_an_unloadable_native_part_leaves_the_python_path(tmp_path, how):
+    src = os.path.dirname(_lib.__file__)
+    pkg = tmp_path / "h3_tp2_amd"
+    shutil.copytree(src, pkg, ignore=shutil.ignore_patterns("__pycache__", "*.so"))
+    for f in os.listdir(src):
+        if f.endswith(".so"):
+            shutil.copy(os.path.join(src, f), pkg / f)
+            if how == "not a library" and f.startswith("_host"):
+                (pkg / f).write_bytes(b"no library")
+    head = "import torch; torch.__version__ = '0.0'; " if how == "another torch" else ""
+    code = head + ("import h3_tp2_amd.ops as o, h3_tp2_amd._lib as l; assert o.__file__.startswith(%r); "
+                   "assert o._host is None; l.load(); print('imported')" % str(pkg))
+    r = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, PYTHONPATH=str(tmp_path)), capture_output=True,
+                       text=True, timeout=300)
+    assert r.returncode == 0 and "imported" in r.stdout, r.stderr
+    assert "native host path does not load" in r.stderr
 
 
 def _bits(out):
