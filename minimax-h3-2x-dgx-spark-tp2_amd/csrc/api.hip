@@ -24,7 +24,7 @@ constexpr int kMaxDevices = 64;
 std::atomic<bool> g_inited[kMaxDevices] = {};
 const uint16_t* g_silu_ptr[kMaxDevices] = {};   // device address of each device's copy of g_h3_silu_table
 const uint16_t* g_silu_rot_ptr[kMaxDevices] = {};   // ... and of g_h3_silu_rot
-int g_cus[kMaxDevices] = {};                    // compute units of each device (persistent GEMM grid size)
+std::atomic<int> g_cus[kMaxDevices] = {};       // compute units of each device (0: not asked yet)
 }  // namespace
 
 namespace h3host {
@@ -168,8 +168,6 @@ int ensure_device_init() {
     if (g_inited[dev].load(std::memory_order_acquire)) return H3FP8_OK;
     std::lock_guard<std::mutex> lock(g_init_mu);
     if (g_inited[dev].load(std::memory_order_relaxed)) return H3FP8_OK;
-    int cus = 0;
-    H3_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     hipStream_t s;
     H3_CHECK_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
     hipLaunchKernelGGL(h3_build_silu_table_kernel, dim3(65536 / 256), dim3(256), 0, s);
@@ -185,17 +183,22 @@ int ensure_device_init() {
     g_silu_rot_ptr[dev] = (const uint16_t*)p;
     const int rc = gemm_scratch_setup(dev);
     if (rc) return rc;
-    g_cus[dev] = cus > 0 ? cus : 1;
     g_inited[dev].store(true, std::memory_order_release);
     return H3FP8_OK;
 }
 
 bool device_ready(int dev) { return dev >= 0 && dev < kMaxDevices && g_inited[dev].load(std::memory_order_acquire); }
 
+// Asked of the device by the first caller, so that entry points that need no set-up choose by it too (a host-side query,
+// also under stream capture).
 int cu_count() {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 1;
-    return g_cus[dev] > 0 ? g_cus[dev] : 1;
+    int cus = g_cus[dev].load(std::memory_order_relaxed);
+    if (cus > 0) return cus;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) return 1;
+    g_cus[dev].store(cus, std::memory_order_relaxed);
+    return cus;
 }
 
 const uint16_t* silu_table_ptr() {

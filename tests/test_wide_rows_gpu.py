@@ -2,10 +2,13 @@
 the oracle's bits at the edges of the forms -- the narrowest row, whole and partial last waves, the row counts on both
 sides of the qkv producer's limit -- and on rows whose fp32 variance depends on the order of the summation, which the four
 waves continue from one to the next."""
+import shutil
+
 import pytest
 import torch
 
 from _util import assert_quant_equal, bits16
+from h3_tp2_amd import _lib, ops
 from oracle import oracle as O
 from test_producers_gpu import EPS, _nan_aware_equal, _order_rows, _tables, mod_inputs
 
@@ -14,7 +17,6 @@ BF16 = torch.bfloat16
 
 
 def _run(cuda, form, x, idx, H, ph=False):
-    from h3_tp2_amd import ops
     M = x.shape[0]
     res, w, sh, sc, gt, _ = mod_inputs(M, H, seed=H + 7)
     gd, shd, scd = _tables(cuda, gt, sh, sc)
@@ -45,6 +47,25 @@ def _run(cuda, form, x, idx, H, ph=False):
 def test_order_sensitive_sums(cuda, form, H):
     x, idx = _order_rows(H)
     _run(cuda, form, x, idx, H)
+
+
+def test_form_rule_before_set_up(cuda, tmp_path):
+    """The producers need no h3fp8_init: a library that has run none (a copy has state of its own) counts the device's
+    compute units all the same, so it takes the same form, and gives the same bits."""
+    lib = _lib.load(shutil.copy(_lib.LIB_PATH, tmp_path / "libh3fp8.so"))
+    assert lib["_ZN6h3host8cu_countEv"]() == torch.cuda.get_device_properties(cuda).multi_processor_count
+    M, H = 100, 5376
+    x, w, sh, sc, gt, _ = mod_inputs(M, H, seed=5)
+    _, shd, scd = _tables(cuda, gt, sh, sc)
+    x, w, idx = x.to(cuda), w.to(cuda), torch.arange(M, device=cuda) % 3
+    q, s = torch.empty((M, H), device=cuda, dtype=torch.float8_e4m3fn), torch.empty((M, 1), device=cuda)
+    rc = lib.h3fp8_rms_quant(x.data_ptr(), H, w.data_ptr(), shd.data_ptr(), shd.stride(0), scd.data_ptr(), scd.stride(0), 3,
+                             idx.data_ptr(), 1, 8, M, H, EPS, q.data_ptr(), H, s.data_ptr(), None, 0,
+                             torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.h3fp8_last_error()
+    q_ref, s_ref = ops.rms_quant(x, w, shd, scd, idx, EPS)
+    torch.cuda.synchronize()
+    assert torch.equal(q.view(torch.uint8), q_ref.view(torch.uint8)) and torch.equal(s, s_ref)
 
 
 @pytest.mark.parametrize("form,M,H", [(f, M, H) for f in ("rms", "gate", "out")
