@@ -426,7 +426,8 @@ __global__ void __launch_bounds__(256) rms_mod_quant_kernel(RmsArgs a) {
 template <bool GATE, int OUT, int CPL, bool B32, bool FULL>
 __global__ void __launch_bounds__(256) rms_mod_quant_wide_kernel(RmsArgs a) {
     __shared__ RowShare share;
-    const int64_t m = blockIdx.x;
+    const int64_t m = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+    if (m >= a.M) return;                               // the whole workgroup
     bool bad0;
     const int64_t i0 = row_index(a, m, bad0);
     rms_mod_quant_row<GATE, OUT, CPL, GATE, B32, FULL, 4>(
@@ -705,9 +706,13 @@ int launch_rms_cpl(const RmsArgs& a, hipStream_t st) {
     return H3FP8_OK;
 }
 
+constexpr int64_t WIDE_GRID_X = 1 << 20;
+
 template <bool GATE, int OUT, int CPL, bool B32>
 int launch_rms_wide(const RmsArgs& a, hipStream_t st) {
-    const dim3 grid((unsigned)a.M), block(256);
+    // a grid dimension holds fewer than 2^32 threads: 2^24 workgroups would not launch
+    const int64_t gx = std::min<int64_t>(a.M, WIDE_GRID_X);
+    const dim3 grid((unsigned)gx, (unsigned)((a.M + gx - 1) / gx)), block(256);
     if (a.H == 4 * 512 * CPL)
         hipLaunchKernelGGL((rms_mod_quant_wide_kernel<GATE, OUT, CPL, B32, true>), grid, block, 0, st, a);
     else

@@ -79,3 +79,28 @@ def test_edges(cuda, form, M, H):
         x[0, H - 1] = float("inf")
         x[1, H // 2] = float("nan")
     _run(cuda, form, x, torch.randint(0, 3, (M,), generator=g), H)
+
+
+def test_more_rows_than_a_grid_dimension_takes(cuda):
+    """2^20 + 5 rows: the launch's second dimension (one dimension of one workgroup per row ends below 2^24).  The rows
+    repeat with a period, in place, with the branch read from the residual's own rows."""
+    period, M, H = 4099, (1 << 20) + 5, 4104
+    tile, w, sh, sc, gt, _ = mod_inputs(period, H, seed=11)
+    gd, shd, scd = _tables(cuda, gt, sh, sc)
+    tile, w = tile.to(cuda), w.to(cuda)
+    rows = torch.arange(M, device=cuda) % period
+    idx = rows % 3
+    u_ref, q_ref, s_ref = ops.gate_rms_quant(tile, gd, tile, w, shd, scd, idx[:period], EPS)
+    x = tile[rows]
+    q, s = torch.empty((M, H), device=cuda, dtype=torch.float8_e4m3fn), torch.empty((M, 1), device=cuda)
+    _lib.call("h3fp8_gate_rms_quant", x.data_ptr(), H, gd.data_ptr(), gd.stride(0), x.data_ptr(), H, w.data_ptr(),
+              shd.data_ptr(), shd.stride(0), scd.data_ptr(), scd.stride(0), 3, idx.data_ptr(), 1, 8, M, H, EPS,
+              x.data_ptr(), H, q.data_ptr(), H, s.data_ptr(), None, 0, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    for r0 in range(0, M, 65536):
+        r = rows[r0:r0 + 65536]
+        assert torch.equal(x[r0:r0 + 65536].view(torch.int16), u_ref[r].view(torch.int16))
+        assert torch.equal(q[r0:r0 + 65536].view(torch.uint8), q_ref.view(torch.uint8)[r])
+        assert torch.equal(s[r0:r0 + 65536].view(torch.int32), s_ref[r].view(torch.int32))
+    del x, q, s
+    torch.cuda.empty_cache()
