@@ -67,8 +67,7 @@ __device__ __forceinline__ uint2 chunk_quant(uint4 v, float inv) {
 template <int CPL, bool KNOWN_AMAX, int WPR = 1, int STORE_AUX = 16>
 __global__ void __launch_bounds__(256) quant_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_t M,
                                                          int64_t K, uint8_t* __restrict__ q, int64_t ldq,
-                                                         float* __restrict__ scale,
-                                                         float* __restrict__ row_amax) {
+                                                         float* scale, float* row_amax) {
     static_assert(WPR == 1 || WPR == 2, "one or two waves per row");
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t row = (int64_t)blockIdx.x * (4 / WPR) + wave / WPR;
@@ -122,9 +121,9 @@ __global__ void __launch_bounds__(256) quant_rows_kernel(const uint16_t* __restr
             __builtin_amdgcn_raw_buffer_store_b64(v2u{o.x, o.y}, qr, (uint32_t)(lane + 64 * j) * 8u, 0, STORE_AUX);
         }
     }
-    if (live && lane == 0) {
-        scale[row] = s;
+    if (live && lane == 0) {                              // the scale last: a caller may pass one array as both
         if (!KNOWN_AMAX && row_amax) row_amax[row] = amax;
+        scale[row] = s;
     }
 }
 

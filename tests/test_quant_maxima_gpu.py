@@ -32,3 +32,22 @@ def test_quant_behind_gemm(cuda, M, N, K, swiglu):
     assert torch.equal(q.view(torch.uint8)[rows], q_ref.view(torch.uint8)[rows])
     assert torch.equal(s.view(-1)[rows], s_ref.view(-1)[rows]) and bool(s[1].isnan().all()) and bool(am[1].isnan())
     assert torch.equal(am[rows], y.float().abs().amax(dim=1)[rows])
+
+
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_workspace_that_is_the_scale_array(cuda, swiglu):
+    """One [M] array as workspace and scale: the scales remain (the maxima are only passed through)."""
+    from h3_tp2_amd import _lib, ops
+    M, N, K = 300, 1040, 256
+    a, w, sa, sb = serving_like(M, 2 * N if swiglu else N, K, seed=7, device=cuda)
+    y = torch.empty((M, N), device=cuda, dtype=torch.bfloat16)
+    q, s = torch.empty((M, N), device=cuda, dtype=E4M3), torch.empty((M, 1), device=cuda)
+    st = torch.cuda.current_stream().cuda_stream
+    head = [a.data_ptr(), K, w.data_ptr(), K, sa.data_ptr(), 1, sb.data_ptr(), 1, None]
+    if swiglu:
+        _lib.call("h3fp8_gemm_swiglu_quant", *head, M, N, K, y.data_ptr(), s.data_ptr(), q.data_ptr(), N, s.data_ptr(), st)
+    else:
+        _lib.call("h3fp8_gemm_quant", *head, y.data_ptr(), N, M, N, K, s.data_ptr(), q.data_ptr(), N, s.data_ptr(), st)
+    q_ref, s_ref = ops.quant_rows(y)
+    torch.cuda.synchronize()
+    assert torch.equal(s, s_ref) and torch.equal(q.view(torch.uint8), q_ref.view(torch.uint8))
