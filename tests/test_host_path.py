@@ -138,6 +138,85 @@ def test_quants_and_producers_match_the_python_path(cuda, monkeypatch):
         _both(monkeypatch, lambda: ops.gate_rms_quant(x, ga[:1], x, w, sh, sc, idx * 0, 1e-6))
 
 
+def _operands(cuda, M=130, N=96, K=272):
+    a, w, sa, sb = int_operands(M, N, K, seed=M, device=cuda)
+    g = torch.Generator(device=cuda).manual_seed(9)
+    x = torch.randn(M, K, generator=g, device=cuda).to(BF16)
+    ada = torch.randn(3, 6 * K, generator=g, device=cuda).to(BF16)
+    norm = torch.randn(K, generator=g, device=cuda).to(BF16)
+    idx = torch.randint(0, 3, (M,), generator=g, device=cuda)
+    bias = torch.randn(N, generator=g, device=cuda).to(BF16)
+    return dict(a=a, w=w, sa=sa, sb=sb, x=x, gate=ada[:, 2 * K:3 * K], sh=ada[:, :K], sc=ada[:, K:2 * K], norm=norm, idx=idx,
+                bias=bias, M=M, N=N, K=K)
+
+
+@pytest.mark.gpu
+def test_takes_the_plain_forms_itself(cuda, monkeypatch):
+    """Called directly, each of the eight functions computes its plain forms (it does not decline them), with the bits of
+    the Python path."""
+    h = _lib.host()
+    o = _operands(cuda)
+    a, w, sa, sb, x, bias = (o[k] for k in ("a", "w", "sa", "sb", "x", "bias"))
+    gate, sh, sc, norm, idx = (o[k] for k in ("gate", "sh", "sc", "norm", "idx"))
+    M, K = o["M"], o["K"]
+    wide = torch.cat((x, x), 1)
+    a_wide = torch.zeros(M, K + 48, device=cuda).to(E4M3)
+    a_wide[:, :K] = a
+    mm = ops.scaled_mm_eligible
+    cases = [("quant_rows", ops.quant_rows, [(x,), (wide[:, :K],), (x[:1],)]),
+             ("gemm", ops.gemm, [(a, w, sa, sb, BF16, None), (a_wide[:, :K], w, sa.view(M, 1), sb.view(1, -1), BF16, bias),
+                                 (a, w, sa[:1], sb[:1].reshape(()), torch.float16, bias.half()),
+                                 (a, w, sa, sb, torch.float32, None), (a[:1], w, sa[:1], sb, BF16, None)]),
+             ("scaled_mm", mm, [(a, w.t(), sa, sb, BF16, None), (a, w.t(), sa.view(M, 1), sb.view(1, -1), BF16, bias),
+                                (a, w.t(), sa[:1], sb, torch.float16, bias.half())]),
+             ("gemm_quant", ops.gemm_quant, [(a, w, sa, sb, None), (a_wide[:, :K], w, sa, sb[:1], bias)]),
+             ("gemm_swiglu_quant", ops.gemm_swiglu_quant, [(a, w, sa, sb, None), (a, w, sa[:1], sb, bias)]),
+             ("silu_mul_quant", ops.silu_mul_quant, [(x,), (wide[:, :K],)]),
+             ("rms_quant", ops.rms_quant, [(x, norm, sh, sc, idx, 1e-6), (wide[:, :K], norm, sh, sc, idx.int(), 1e-6)]),
+             ("gate_rms_quant", ops.gate_rms_quant, [(x, gate, wide[:, K:], norm, sh, sc, idx, 1e-6)])]
+    monkeypatch.setattr(ops, "_host", None)                    # the functions of ops below: the Python path
+    assert len(cases) == 8
+    for name, python, forms in cases:
+        for args in forms:
+            got = getattr(h, name)(*args)
+            assert got is not None, (name, [getattr(t, "shape", t) for t in args])
+            ref = python(*args)
+            got, ref = _bits(got), _bits(ref)
+            assert [g[:3] for g in got] == [r[:3] for r in ref], name
+            assert all(torch.equal(g[3], r[3]) for g, r in zip(got, ref)), name
+
+
+@pytest.mark.gpu
+def test_declines_what_python_checks(cuda):
+    h = _lib.host()
+    o = _operands(cuda)
+    a, w, sa, sb, x, bias = (o[k] for k in ("a", "w", "sa", "sb", "x", "bias"))
+    gate, sh, sc, norm, idx = (o[k] for k in ("gate", "sh", "sc", "norm", "idx"))
+    strided = torch.stack((bias, bias), 1)[:, 0]
+    for ops4 in ((a, w, sa.double(), sb), (a, w, sa, sb[:-1]), (a.float(), w, sa, sb), (a, w[:, :-16], sa, sb),
+                 (a.t().contiguous().t(), w, sa, sb), (a.cpu(), w, sa, sb), (a, w.cpu(), sa, sb), (a[:0], w, sa[:0], sb)):
+        assert h.gemm(*ops4, BF16, None) is None and h.gemm_quant(*ops4, None) is None
+        assert h.gemm_swiglu_quant(*ops4, None) is None
+        assert h.scaled_mm(ops4[0], ops4[1].t(), *ops4[2:], BF16, None) is None
+    for b in (strided, bias.half(), bias[:-1], bias.view(1, -1), bias.cpu()):
+        assert h.gemm(a, w, sa, sb, BF16, b) is None and h.scaled_mm(a, w.t(), sa, sb, BF16, b) is None
+        assert h.gemm_quant(a, w, sa, sb, b) is None and h.gemm_swiglu_quant(a, w, sa, sb, b) is None
+    assert h.gemm(a, w, sa, sb, torch.float32, bias) is None and h.gemm(a, w, sa, sb, torch.float64, None) is None
+    assert h.scaled_mm(a, w.t(), sa[:1], sb[:1], BF16, None) is None         # per-tensor scales on both sides
+    assert h.scaled_mm(a, w.t(), sa, sb, torch.float32, None) is None
+    assert h.scaled_mm(a, w.t().contiguous(), sa, sb, BF16, None) is None
+    assert h.gemm_swiglu_quant(a, w[:-1], sa, sb[:-1], None) is None         # an odd number of gate | up rows
+    for t in (x.float(), x[0], x.t(), x[:, ::2], x[:0], x.cpu()):
+        assert h.quant_rows(t) is None and h.silu_mul_quant(t) is None
+    assert h.silu_mul_quant(x[:, :-4]) is None
+    for args in ((x, norm.view(1, -1), sh, sc, idx, 1e-6), (x, norm, sh[:, :-8], sc, idx, 1e-6),
+                 (x, norm, sh, sc.float(), idx, 1e-6), (x, norm, sh, sc, idx.float(), 1e-6), (x, norm, sh, sc, idx[:-1], 1e-6),
+                 (x, norm, sh, sc, idx, 1)):
+        assert h.rms_quant(*args) is None
+        assert h.gate_rms_quant(args[0], gate, x, *args[1:]) is None
+    assert h.gate_rms_quant(x, gate, x[:-1], norm, sh, sc, idx, 1e-6) is None
+
+
 @pytest.mark.gpu
 def test_runs_on_the_current_stream_and_under_capture(cuda):
     a, w, sa, sb = int_operands(40, 96, 256, seed=1, device=cuda)
@@ -145,9 +224,10 @@ def test_runs_on_the_current_stream_and_under_capture(cuda):
     x = torch.randn(40, 256, device=cuda).to(BF16)
     q_ref, s_ref = ops.quant_rows(x)
     graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
-        y = ops.gemm(a, w, sa, sb)
-        q, s = ops.quant_rows(x)
+    h = _lib.host()
+    with torch.cuda.graph(graph):                              # the native functions themselves: None would not unpack
+        y = h.gemm(a, w, sa, sb, BF16, None)
+        q, s = h.quant_rows(x)
     for _ in range(3):
         y.zero_()
         s.zero_()
