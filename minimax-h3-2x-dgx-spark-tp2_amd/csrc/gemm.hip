@@ -1020,18 +1020,30 @@ Split split_for(const GemmParams& p, int panels, bool swiglu, int G) {
     return s;
 }
 
-int launch_split(GroupedParams gp, int epi, int out_dt, bool has_bias, hipStream_t st) {
-    GemmParams& p = gp.g[0];
-    const int G = h3host::cu_count();
+// How a problem runs: in one smaller form as a whole (form < TILE_FORMS), else by the split.
+struct Plan {
+    int form;
+    Split split;
+};
+
+Plan plan_for(const GemmParams& p, bool swiglu, int G) {
     const int nk = (p.K + BK - 1) / BK;
-    const bool swiglu = epi == EPI_SWIGLU;
-    const int form = tile_form_for(p.M, p.w_rows, swiglu, G);
-    if (form < TILE_FORMS) return launch_tiles(p, form, out_dt, swiglu, st);
-    Split s = split_for(p, p.tiles_m, swiglu, G);
+    Plan plan{tile_form_for(p.M, p.w_rows, swiglu, G), {}};
+    if (plan.form < TILE_FORMS) return plan;
+    plan.split = split_for(p, p.tiles_m, swiglu, G);
     if (p.M % BM != 0 && p.M > BM) {
         const Split whole = split_for(p, p.tiles_m - 1, swiglu, G);
-        if (whole.form < TILE_FORMS && split_cost(whole, nk, G) < split_cost(s, nk, G)) s = whole;
+        if (whole.form < TILE_FORMS && split_cost(whole, nk, G) < split_cost(plan.split, nk, G)) plan.split = whole;
     }
+    return plan;
+}
+
+int launch_split(GroupedParams gp, int epi, int out_dt, bool has_bias, hipStream_t st) {
+    GemmParams& p = gp.g[0];
+    const bool swiglu = epi == EPI_SWIGLU;
+    const Plan plan = plan_for(p, swiglu, h3host::cu_count());
+    if (plan.form < TILE_FORMS) return launch_tiles(p, plan.form, out_dt, swiglu, st);
+    const Split& s = plan.split;
     p.tiles_m = s.panels;
     gp.total_tiles = s.full;
     const int rc = s.full == 0        ? H3FP8_OK
@@ -1140,6 +1152,19 @@ int quant_rows_max_launch(const void* x, int64_t ldx, int64_t M, int64_t K, floa
                           float* scale, hipStream_t st);
 int quant_args_ok(const void* x, int64_t ldx, int64_t M, int64_t K, const void* q, int64_t ldq, const float* scale);
 }
+
+namespace h3host {
+// The plan of one launch over M > 32 rows on G CUs, for the tests (host only): the form that runs the whole problem, then
+// the split's row panels, full tiles, tiles left and tail form; TILE_FORMS stands for none.  swiglu: N is F.
+void gemm_plan(int64_t M, int64_t N, int64_t K, int swiglu, int G, int* out) {
+    const GemmParams p = make_params(nullptr, K, nullptr, K, nullptr, 1, nullptr, 1, nullptr, nullptr, N, M, N, K,
+                                     swiglu ? 2 * N : N, nullptr, nullptr, swiglu != 0);
+    const Plan plan = plan_for(p, swiglu != 0, G);
+    const Split s = plan.form < TILE_FORMS ? Split{0, 0, 0, TILE_FORMS} : plan.split;
+    const int v[5] = {plan.form, s.panels, s.full, s.rest, s.form};
+    std::copy(v, v + 5, out);
+}
+}  // namespace h3host
 
 // Rows up to this width: the quant behind a GEMM holds its row in registers and reduces the row maxima itself (it writes
 // them to the workspace), since that costs it nothing (91 728 x 8192: 354 us, with the maxima given 353; x 3072: 124 and

@@ -143,6 +143,7 @@ bool device_ready(int dev);                    // has ensure_device_init complet
 int gemm_scratch_setup(int dev);               // the device address of gemm.hip's row-maxima buffer (set-up only)
 const uint16_t* silu_table_ptr();              // device address of the current device's SiLU table
 const uint16_t* silu_rot_ptr();                // ... and of its compact rotated-key copy (kernel 3's LDS table)
+void gemm_plan(int64_t M, int64_t N, int64_t K, int swiglu, int G, int* out);   // gemm.hip: how a GEMM runs
 int cu_count();                                // compute units of the current device (needs no set-up)
 }  // namespace h3host
 

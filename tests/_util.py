@@ -65,6 +65,24 @@ def serving_like(M: int, N: int, K: int, seed: int, device):
     return a.to(device), wq.to(device), torch.from_numpy(sa).to(device), torch.from_numpy(sw).to(device)
 
 
+FORMS = ((32, 64), (64, 64), (96, 64), (128, 64), (128, 128), (192, 128), (256, 128))   # smaller tiles: weight x token rows
+
+
+def gemm_plan(M: int, N: int, K: int, swiglu: bool = False, cus: int = 256) -> dict:
+    """What the library runs for one launch of M > 32 rows (its own rule, csrc/gemm.hip): ``form`` of the whole problem or
+    None, else the full tiles' ``panels`` of 256 token rows and their number ``full``, the ``rest`` of those panels' tiles
+    that the tail takes, and the tail's form or None.  swiglu: N = F."""
+    import ctypes
+
+    from h3_tp2_amd import _lib
+    out = (ctypes.c_int * 5)()
+    i64 = ctypes.c_int64
+    _lib.load()["_ZN6h3host9gemm_planEllliiPi"](i64(M), i64(N), i64(K), int(swiglu), cus, out)
+    form, panels, full, rest, tail = out
+    none = len(FORMS)
+    return dict(form=None if form == none else form, panels=panels, full=full, rest=rest, tail=None if tail == none else tail)
+
+
 def ref_gemm(a: torch.Tensor, w: torch.Tensor, sa, sb, bias=None, out_fp16=False) -> np.ndarray:
     """oracle: fp32 product of the e4m3 codes (numpy BLAS) + the scaled epilogue -> output bit patterns."""
     acc = O.matmul_f32(bits8(a), bits8(w))

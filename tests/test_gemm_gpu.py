@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 import torch
 
-from _util import (ACC_REL, abs_products, assert_quant_equal, bits8, bits16, check_close_bf16, gemm_acc_err,
+from _util import (ACC_REL, abs_products, assert_quant_equal, bits8, bits16, check_close_bf16, gemm_acc_err, gemm_plan,
                    int_operands, oracle_quant, ref_gemm, serving_like)
 from oracle import oracle as O
 
@@ -56,11 +56,14 @@ def test_integer_inputs_exact_with_guards(cuda, M, N, K):
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("scalar", ["none", "sa", "sb"])
-@pytest.mark.parametrize("N", [528, 400])
-def test_integer_inputs_dtypes_bias_scalars(cuda, out_dtype, bias, scalar, N):
-    """Output dtypes, bias and scalar scales, exact on integer operands; N = 528 runs as 12 half tiles, N = 400 as
-    9 tiles of 128 x 192 (ragged in both M and N)."""
-    M, K = 300, 768
+@pytest.mark.parametrize("M,N,K", [(300, 528, 768), (300, 400, 768), (777, 3072, 144), (2040, 2992, 256), (2300, 3600, 96),
+                                   (4100, 4368, 64)])
+def test_integer_inputs_dtypes_bias_scalars(cuda, out_dtype, bias, scalar, M, N, K):
+    """Output dtypes, bias and scalar scales, exact on integer operands, ragged in M and N: tiles of 32 x 64 (two shapes),
+    128 x 128 and 192 x 128, full tiles only (135) and a whole round of full tiles with a tail of 128 x 128."""
+    p = gemm_plan(M, N, K)
+    assert (p["form"], p["full"], p["tail"]) == {777: (4, 0, None), 2040: (5, 0, None), 2300: (None, 135, None),
+                                                 4100: (None, 256, 4)}.get(M, (0, 0, None))
     a, w, sa, sb = int_operands(M, N, K, seed=11, device=cuda)
     if scalar == "sa":
         sa = sa[:1].reshape(())
@@ -96,9 +99,8 @@ def test_measured_shapes_within_tolerance(cuda, name):
 
 @pytest.mark.parametrize("M,N,K", [(777, 3072, 1024), (4100, 4368, 256), (2300, 3600, 256)])
 def test_fused_row_amax_and_quant(cuda, M, N, K):
-    """The fused next-layer quant: the row maxima and the quant from them equal the plain GEMM's output and kernel 1 on
-    it, for 128 x 192 tiles (48 full tiles run as 112 of these), whole rounds plus a half-tile tail (306) and full tiles
-    only (135)."""
+    """The row maxima from the epilogue and the quant behind the GEMM equal the plain GEMM's output and kernel 1 on it, for
+    128 x 128 tiles, a whole round plus a tail of these (256 full tiles of 306) and full tiles only (135)."""
     from h3_tp2_amd import ops
     a, w, sa, sb = serving_like(M, N, K, seed=3 + M, device=cuda)
     amax = torch.full((M,), 123.0, device=cuda)          # the library zeroes it first
@@ -208,10 +210,10 @@ def test_accumulator_error_model(cuda, kind, M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [(16740, 9216, 3072), (2048, 3072, 3072), (31248, 3072, 1024)])
 def test_half_tile_tail_equals_full_tiles(cuda, M, N, K):
-    """A launch whose last round runs as half tiles (256 x 128), or whose whole problem runs as 128 x 192 tiles (2048 x
-    3072: 256 of them), gives the same bits as all full tiles (the grouped path never splits): the same MFMA sequence
-    per output element.  Also the fused row maxima + quant through the split launch against the oracle's quant of its
-    own output."""
+    """A launch whose last round runs in smaller tiles (128 x 128 at M = 16 740), whose whole problem runs as 192 x 128
+    tiles (2048 x 3072: 256 of them) or all of whose rounds are full tiles (31 248) gives the same bits as all full tiles
+    (the grouped path never splits): the same MFMA sequence per output element.  Also the quant behind the split launch
+    against the oracle's quant of its own output."""
     from h3_tp2_amd import ops
     a, w, sa, sb = serving_like(M, N, K, seed=7, device=cuda)
     y = _gemm(a, w, sa, sb)
@@ -227,10 +229,10 @@ def test_half_tile_tail_equals_full_tiles(cuda, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(4096, 4352, 128), (4100, 4368, 64), (5000, 2560, 64), (2300, 3600, 192),
                                    (1000, 3008, 96), (6000, 2816, 48), (2048, 4096, 64), (300, 400, 176)])
 def test_integer_inputs_exact_launch_splits(cuda, M, N, K):
-    """Shapes whose tile counts take each launch form on 256 CUs: whole rounds plus a half-tile tail (272, 306 and 264
-    tiles), full tiles only (200 and 135 tiles), half tiles only (128 tiles), 128 x 192 tiles (48 full tiles as 128
-    of these; 4 as 9, ragged in M, N and K); K below one 128-deep k-step; integer operands, so the output must equal
-    the oracle bit for bit, with guard sentinels around it."""
+    """Shapes whose tile counts take each launch form on 256 CUs: a whole round plus a tail (272 tiles: 64 x 64, 306: 128 x
+    128, 264: 32 x 64), full tiles only (200 and 135 tiles), smaller tiles only (2048 x 4096: 256 x 128, 1000 x 3008: 128 x
+    128, 300 x 400: 32 x 64, ragged in M, N and K); K below one 128-deep k-step; integer operands, so the output must
+    equal the oracle bit for bit, with guard sentinels around it."""
     from h3_tp2_amd import ops
     a, w, sa, sb = int_operands(M, N, K, seed=7 * M + N + K, device=cuda)
     ref = ref_gemm(a, w, sa, sb)

@@ -1,12 +1,11 @@
 """Race stress of the GEMM kernels' hand-rolled stage release (fence-free barriers with explicit vmcnt / lgkmcnt waits):
-kernel 2 at the 960x576 QKV shape (full tiles with the half-tile tail), kernel 3 at the 1344x768 FFN gate/up shape,
-the single linear 2048 x 3072 x 3072 (the 128 x 192 tiles: a three-stage ring with one barrier per k-step) and the
-M = 2 adaLN GEMM 2 x 3072 -> 18 432 (the small-M form: a per-wave LDS ring released by its own vmcnt / lgkmcnt waits
-alone), launched again and again while a
-memory-bound co-runner (a 1 GiB device-to-device copy) runs on a second stream of the same (default) priority, so that
-the persistent workgroups meet unpredictable memory latencies and CU sharing.  Every output must equal the first one
-bit for bit (and the first must equal a launch with no co-runner).  The loop stops at the first mismatch and is
-bounded in time.  A LDS stage refilled before every wave finished reading it, or read before its loads landed, shows
+kernel 2 at the 960x576 QKV shape (full tiles with a tail of 128 x 128), kernel 3 at the 1344x768 FFN gate/up shape,
+the single linear 2048 x 3072 x 3072 (192 x 128 tiles: a three-stage ring with one barrier per k-step) and the M = 2
+adaLN GEMM 2 x 3072 -> 18 432 (the small-M form: a per-wave LDS ring released by its own vmcnt / lgkmcnt waits alone),
+launched again and again while a memory-bound co-runner (a 1 GiB device-to-device copy) runs on a second stream of the
+same (default) priority, so that the persistent workgroups meet unpredictable memory latencies and CU sharing.  Every
+output must equal the first one bit for bit (and the first must equal a launch with no co-runner).  The loop stops at
+the first mismatch and is bounded in time.  A LDS stage refilled before every wave finished reading it, or read before its loads landed, shows
 up here as a differing output under load -- the failure the reference found in its own kernel
 (results/20261103-cutlass-sm120/race.md, scripts/fp8_cutlass_stress.py).
 
@@ -49,7 +48,7 @@ def run(seconds: float, device, log=print) -> dict:
     ref2 = ops.gemm(a2, w2, s2, sw2)
     ref3 = ops.gemm_swiglu(a3, w3, s3, sw3, row_amax=amax3)
     ref_amax3 = amax3.clone()
-    ref1 = ops.gemm(a1, w1, s1, sw1)                        # 256 tiles of 128 x 192
+    ref1 = ops.gemm(a1, w1, s1, sw1)                        # 256 tiles of 192 x 128
     ref4 = ops.gemm(a4, w4, s4, sw4)                        # the small-M form
     out1, out4 = torch.empty_like(ref1), torch.empty_like(ref4)
     torch.cuda.synchronize()
