@@ -1004,7 +1004,7 @@ struct Split {
 // (measured: 101 tiles as 202 of 256 x 128, 56 k-steps, 44 us; 112 x 4 rows as 224 of 128 x 64, 42 k-steps, 25-27 us,
 // with their weights from HBM).
 int64_t split_cost(const Split& s, int nk, int G) {
-    constexpr int kTailStep[TILE_FORMS + 1] = {180, 200, 250, 290, 420, 600, 700, 0};
+    constexpr int kTailStep[TILE_FORMS] = {180, 200, 0, 290, 420, 0, 700};   // 96 and 192 rows do not divide a full tile
     return (int64_t)((s.full + G - 1) / G) * (1350LL * nk + 5000) +
            (s.form < TILE_FORMS ? (int64_t)kTailStep[s.form] * nk + 6000 : 0);
 }

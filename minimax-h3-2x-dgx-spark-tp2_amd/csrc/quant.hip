@@ -127,12 +127,13 @@ __global__ void __launch_bounds__(256) quant_rows_kernel(const uint16_t* __restr
     }
 }
 
-// Rows too wide for the register-resident form: the row is read twice (max pass, then quant pass).
+// Rows too wide for the register-resident form (more than 16 384 columns): the row is read twice (max pass, then quant
+// pass).
 template <bool KNOWN_AMAX>
 __global__ void __launch_bounds__(256) quant_rows_wide_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_t M,
                                                               int64_t K, uint8_t* __restrict__ q, int64_t ldq,
                                                               float* __restrict__ scale,
-                                                              float* __restrict__ row_amax) {
+                                                              const float* __restrict__ row_amax) {
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= M) return;
@@ -153,10 +154,7 @@ __global__ void __launch_bounds__(256) quant_rows_wide_kernel(const uint16_t* __
     const float inv = inv_scale(s);
     uint2* qr = reinterpret_cast<uint2*>(q + row * ldq);
     for (int64_t c = lane; c < nchunk; c += 64) qr[c] = chunk_quant<false>(xr[c], inv);
-    if (lane == 0) {
-        scale[row] = s;
-        if (!KNOWN_AMAX && row_amax) row_amax[row] = amax;
-    }
+    if (lane == 0) scale[row] = s;
 }
 
 template <bool KNOWN>
@@ -293,10 +291,12 @@ int quant_rows_amax_launch(const void* x, int64_t ldx, int64_t M, int64_t K, con
     return launch_quant<true>(x, ldx, M, K, q, ldq, scale, const_cast<float*>(row_amax), st);   // only read
 }
 
+// Writes the row maxima as well, on rows that the register-resident form takes.
 int quant_rows_max_launch(const void* x, int64_t ldx, int64_t M, int64_t K, float* row_amax, void* q, int64_t ldq,
                           float* scale, hipStream_t st) {
     int rc = check_quant_args(x, ldx, M, K, q, ldq, scale);
     if (rc) return rc;
+    H3_REQUIRE(K <= 32 * 512, "quant: K=%lld is too wide for the form that stores its row maxima", (long long)K);
     return launch_quant<false>(x, ldx, M, K, q, ldq, scale, row_amax, st);
 }
 }  // namespace h3host
