@@ -989,10 +989,10 @@ int dispatch(const GroupedParams& gp, int out_dt, bool has_bias, hipStream_t st)
 //     one launch of smaller tiles (a tail) for what that leaves: the last partial round's tiles, and the ragged rows as
 //     the few tiles that they fill.  A tail takes the smallest form whose tiles fit one round.  Where none does, the full
 //     tiles cover all panels and the last round runs partly filled.  The cheaper of the two by split_cost.
-//     Against full tiles over all panels and a tail of four-wave 256 x 128 tiles for at most G / 2 tiles left:
-//     4100 x 5376 x 14336 255.0 -> 242.6 us (101 tiles left), 16 740 x 9216 x 3072 372.7 -> 364.1 (72 left).  With the
-//     4 ragged rows of 4100 left to the tail: an H3 MLP behind the stock fc1 (7 rounds + 112 tiles of 4 rows, instead of
-//     7.4 rounds) 826 -> 811 us.
+//     Against full tiles over all panels and a tail of four-wave 256 x 128 tiles for at most G / 2 tiles left, the GEMM
+//     alone: 4100 x 5376 x 14336 255.0 -> 242.6 us (101 tiles left), 16 740 x 9216 x 3072 372.7 -> 364.1 (36 left, and the
+//     ragged rows; with its producer in front 418 -> 414, within the noise).  With the 4 ragged rows of 4100 left to the
+//     tail: an H3 MLP behind the stock fc1 (7 rounds + 112 tiles of 4 rows, instead of 7.4 rounds) 826 -> 811 us.
 struct Split {
     int panels;                // row panels that the full tiles cover
     int full, rest;            // full tiles launched, tiles of those panels left to the tail

@@ -13,8 +13,9 @@
 // two k-steps; the large ones are bound by the fragment reads of their waves (LDS returns 95 bytes per cycle to one
 // wave per SIMD, 250 to two), so they run two waves per SIMD.  Measured against the forms before (128 x 192 and 256 x
 // 128 tiles of four waves), M x N x K, operands in the MALL: 64 x 5376 x 14336 71.0 -> 20.9 us, 200 x 5376 x 14336 69.6
-// -> 29.2, 512 x 6144 x 4096 24.6 -> 16.9, 2048 x 3072 x 3072 23.5 -> 21.4, 1000 x 5376 x 14336 81.8 -> 67.5, 768 x
-// 9216 x 3072 28.9 -> 23.2.
+// -> 29.2 (weights from HBM 83.8 -> 39.7), 512 x 6144 x 4096 24.6 -> 16.9, 2048 x 3072 x 3072 23.5 -> 21.4 (behind its
+// quant, both 28.6 -> 28.2: within the noise), 1000 x 5376 x 14336 81.8 -> 67.5 (weights from HBM: 79, the MLP around it
+// 242 -> 237), 768 x 9216 x 3072 28.9 -> 23.2.
 #include "gemm_core.h"
 
 namespace {
