@@ -209,7 +209,7 @@ def test_accumulator_error_model(cuda, kind, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(16740, 9216, 3072), (2048, 3072, 3072), (31248, 3072, 1024)])
-def test_half_tile_tail_equals_full_tiles(cuda, M, N, K):
+def test_split_launch_equals_full_tiles(cuda, M, N, K):
     """A launch whose last round runs in smaller tiles (128 x 128 at M = 16 740), whose whole problem runs as 192 x 128
     tiles (2048 x 3072: 256 of them) or all of whose rounds are full tiles (31 248) gives the same bits as all full tiles
     (the grouped path never splits): the same MFMA sequence per output element.  Also the quant behind the split launch

@@ -5,7 +5,8 @@ asm the compiler puts none.
   32x32x64 on 8-bit operands needs 20; 24 is what the kernels put there, so a smaller gap has come in before them);
 * an LDS-DMA load (buffer_load ... lds) comes at least one wait state behind the scalar instruction that wrote M0, its LDS
   address;
-* a memory instruction reads scalar registers that a vector instruction wrote at least five wait states before.
+* a memory instruction reads scalar registers that a vector instruction wrote at least five wait states before;
+* a lane move (DPP, permlane swap) reads a register at least two wait states behind the vector instruction that wrote it.
 
 A wait state is one issued instruction, s_nop n counts n + 1; every path through branches and loops is followed.
 """
@@ -22,6 +23,7 @@ OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
 MFMA_STATES = 24
 M0_STATES = 1
 SGPR_STATES = 5
+LANE_STATES = 2
 
 
 def _code_objects(path):
@@ -147,6 +149,16 @@ def sgpr_gaps(insns):
     return out
 
 
+def lane_gaps(insns):
+    """The lane moves too close behind a vector instruction that wrote the register they move."""
+    moves = {i: _vregs(args if "permlane" in op else args.split(", ")[1].split()[0])
+             for i, (op, args, _) in enumerate(insns) if "permlane" in op or op.endswith("_dpp")}
+    if not moves:
+        return []
+    return [j for i, (op, args, _) in enumerate(insns) if op.startswith("v_") and not op.startswith("v_cmp")
+            for j in _within(insns, i, LANE_STATES) if j in moves and _vregs(args.split(", ")[0]) & moves[j]]
+
+
 @pytest.fixture(scope="module")
 def kernels(tmp_path_factory):
     assert os.path.exists(OBJDUMP), "the ROCm toolchain that builds the library has no llvm-objdump"
@@ -173,6 +185,11 @@ def test_m0_is_written_early_enough(kernels):
 
 def test_scalar_registers_are_written_early_enough(kernels):
     bad = {k: len(g) for k, g in ((k, sgpr_gaps(ins)) for k, ins in kernels.items()) if g}
+    assert not bad, bad
+
+
+def test_lanes_move_late_enough(kernels):
+    bad = {k: len(g) for k, g in ((k, lane_gaps(ins)) for k, ins in kernels.items()) if g}
     assert not bad, bad
 
 
@@ -214,3 +231,11 @@ def test_finds_a_descriptor_right_behind_its_writer():
     assert sgpr_gaps(_insns(write, "s_nop 3", _LOAD)) == [2]
     assert sgpr_gaps(_insns(write, "s_nop 4", _LOAD)) == []
     assert sgpr_gaps(_insns("s_nop 0", _LOAD, write, "s_nop 2", ("s_cbranch_scc1 65532", 1), "s_endpgm")) == [1]
+
+
+def test_finds_a_lane_move_right_behind_its_writer():
+    write = "v_maximum3_f32 v3, v3, |v4|, |v5|"
+    dpp, swap = "v_mov_b32_dpp v6, v3 row_shl:8 row_mask:0xf bank_mask:0xf", "v_permlane32_swap_b32_e32 v7, v3"
+    assert lane_gaps(_insns(write, "s_nop 0", dpp)) == [2] and lane_gaps(_insns(write, "s_nop 1", dpp)) == []
+    assert lane_gaps(_insns(write, swap)) == [1] and lane_gaps(_insns(write, "s_nop 1", swap)) == []
+    assert lane_gaps(_insns(write, "v_mov_b32_dpp v6, v4 row_shl:8 row_mask:0xf bank_mask:0xf")) == []
